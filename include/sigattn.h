@@ -144,6 +144,21 @@ int sigattn_fwd_ws(const sigattn_problem *p, void *out, void *workspace, size_t 
                    void *stream);
 
 /*
+ * sigattn_fwd_ws with a finer plan for long or many key caches (no
+ * counterpart in the reference): a split-KV problem large enough to give
+ * every wave of the GPU a chunk of its own (256 keys or more) runs that way,
+ * the waves of a workgroup on neighbouring heads, with
+ * sigattn_fwd_decode_workspace_bytes(p) bytes of partials; every other
+ * problem runs, and asks for, exactly what sigattn_fwd_ws does.  Deterministic,
+ * and equal to sigattn_fwd_ws within fp32 summation order.  With workspace
+ * NULL it is sigattn_fwd; a workspace smaller than the partials returns
+ * SIGATTN_ERR_WORKSPACE.
+ */
+size_t sigattn_fwd_decode_workspace_bytes(const sigattn_problem *p);
+int sigattn_fwd_decode(const sigattn_problem *p, void *out, void *workspace, size_t workspace_bytes,
+                       void *stream);
+
+/*
  * sigattn_fwd_ws without a caller workspace and without any allocation
  * (no counterpart in the reference): for callers that cannot allocate device
  * memory -- code under HIP graph capture, tight serving loops, harnesses that

@@ -160,3 +160,58 @@ def test_decode_long_cache_sum_of_halves():
     h1, h2 = f(k[:, :Tk // 2], v[:, :Tk // 2]), f(k[:, Tk // 2:], v[:, Tk // 2:])
     mag = max(t.abs().max().item() for t in (whole, h1, h2))
     torch.testing.assert_close(whole, h1 + h2, atol=3 * 2 ** -8 * mag, rtol=0)
+
+
+@pytest.mark.parametrize("B,H,Tq,Tk,D,packed,mod", [
+    (8, 16, 1, 2100, 64, False, False),    # 9 chunks of 256, the last short
+    (10, 13, 3, 2111, 128, False, True),   # units not a multiple of the workgroup's four
+    (8, 16, 32, 8200, 64, False, True),    # all 32 query rows; chunks of 1088
+    (9, 16, 2, 3001, 128, True, True),     # packed rows
+    (16, 128, 2, 300, 64, False, False),   # one chunk per (batch, head): no partials
+])
+def test_decode_wave_per_chunk_matches_the_general_path(B, H, Tq, Tk, D, packed, mod):
+    """sigattn_fwd_decode's plan (a wave per chunk) against sigattn_fwd_ws and
+    the oracle: ragged and empty caches, short last chunks and blocks."""
+    lib = _capi.load_library()
+    g = torch.Generator().manual_seed(B * Tk + D)
+    lens = torch.randint(1, Tk + 1, (B,), generator=g)
+    lens[0], lens[1], lens[2] = Tk, 0, 33
+    rows = int(lens.sum())
+    q = randn((B * Tq, H, D) if packed else (B, Tq, H, D), torch.bfloat16, DEV, g)
+    k, v = (randn((rows, H, D) if packed else (B, Tk, H, D), torch.bfloat16, DEV, g) for _ in range(2))
+    sm = torch.randn((rows,) if packed else (B, Tk), generator=g).to(DEV) if mod else None
+    bias = torch.full((B,), -3.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    cu_q = (torch.arange(B + 1) * Tq).to(DEV, torch.int32)
+    cu_k = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).to(DEV, torch.int32)
+    sq = torch.full((B,), Tq, dtype=torch.int32, device=DEV)
+    sk = lens.to(DEV, torch.int32)
+    if packed:
+        pr = _capi._problem(q, k, v, bias, sm, scale, None, None, False, packed=(cu_q, cu_k, Tq, Tk))
+    else:
+        pr = _capi._problem(q, k, v, bias, sm, scale, sq, sk, False)
+    stream = torch.cuda.current_stream().cuda_stream
+    outs = []
+    for size, run in ((lib.sigattn_fwd_decode_workspace_bytes, lib.sigattn_fwd_decode),
+                      (lib.sigattn_fwd_workspace_bytes, lib.sigattn_fwd_ws)):
+        n = size(ctypes.byref(pr))
+        ws = torch.full((max(n, 1),), 255, dtype=torch.uint8, device=DEV)  # NaN bytes
+        o = torch.full_like(q, float("nan"))
+        assert run(ctypes.byref(pr), o.data_ptr(), ws.data_ptr(), n, stream) == 0
+        outs.append(o.view(B, Tq, H, D))
+    torch.cuda.synchronize()
+    # One rounding to bf16 of sums in another order: at most one bf16 step of the largest value.
+    torch.testing.assert_close(outs[0], outs[1], atol=2 ** -7 * outs[1].abs().max().item(), rtol=0)
+    heads = slice(0, H, max(1, H // 2))
+    qs = q.view(B, Tq, H, D)
+    for b in range(min(B, 4)):
+        n, first = int(lens[b]), int(cu_k[b])
+        ks, vs = (t[first:first + n] if packed else t[b, :n] for t in (k, v))
+        if n == 0:
+            assert torch.all(outs[0][b] == 0)
+            continue
+        ms = None if sm is None else (sm[first:first + n] if packed else sm[b, :n])[None]
+        want, _ = oracle_fwd_bwd(qs[b:b + 1, :, heads], ks[None, :, heads], vs[None, :, heads], None,
+                                 scale=np.float32(1 / math.sqrt(D)), bias=np.full(1, -3.0), score_mod=ms,
+                                 with_bwd=False)
+        assert_close_to_oracle(outs[0][b:b + 1, :, heads], want, torch.bfloat16, f"sequence {b}")

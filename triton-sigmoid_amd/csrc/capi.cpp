@@ -98,7 +98,7 @@ bool use_f32_mfma(const sigattn_problem *p, const void *const *ptrs, int nptr) {
 // decode shapes, targets from 256 to 2048 workgroups run within noise of each
 // other; 512 keeps the partials small.
 struct SplitPlan {
-  int nsplit = 0, chunk = 0;
+  int nsplit = 0, chunk = 0, unit_waves = 4;
 };
 
 #ifndef SIGATTN_SPLIT_TARGET
@@ -122,6 +122,36 @@ SplitPlan splitkv_plan(const sigattn_problem *p, bool mfma) {
   const int64_t chunk = cdiv(cdiv(p->Tk, n), 128) * 128;
   sp.nsplit = (int)cdiv(p->Tk, chunk);
   sp.chunk = (int)chunk;
+  return sp;
+}
+
+// The plan that reads the caches fastest: a wave per (batch, head, chunk)
+// (launch_fwd_splitkv's unit_waves = 1) where chunks of 256 keys would give
+// every SIMD a wave of its own (four per CU), with chunks for about eight
+// waves per CU; nsplit = 0 elsewhere, where four waves share a chunk (at a
+// quarter of the key range each: B=4 H=32 D=64 Tk=2000, 4 chunks of 512, takes
+// the same time either way, 30 us, most of it host time).  Eight, because
+// every unit starts with two round trips to memory and the units of a round
+// start together, while fewer chunks leave ragged caches uneven.  Waves per CU
+// 4 / 8 / 16 / 32, us: B=16 H=32 D=128 Tk=8192 full 319 / 323 / 366 / 412,
+// lengths 1186..8192 199 / 195 / 198 / 197, B=32 H=32 D=64 Tq=4 Tk=4096 214 /
+// 167 / 171 / 176, B=12 H=12 D=64 Tq=8 lengths 800..6001 49 / 37 / 41 / 41.
+constexpr int64_t kDecodeChunk = 256, kDecodeMinWaves = 4, kDecodeWaves = 8;
+SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
+  SplitPlan sp = splitkv_plan(p, mfma);
+  if (sp.nsplit == 0) return sp;
+  const int64_t cus = sigattn::device_compute_units(), pairs = p->B * p->H;
+  // The partials (written and read, 8·Tq·D bytes a chunk) stay below an eighth
+  // of the K and V they come from (4·D bytes a key).
+  const int64_t least = kDecodeChunk > 32 * p->Tq ? kDecodeChunk : 32 * p->Tq;
+  const int64_t most = cdiv(p->Tk, least);
+  if (cus <= 0 || pairs * most < kDecodeMinWaves * cus) return SplitPlan{};
+  int64_t n = cdiv(kDecodeWaves * cus, pairs);
+  if (n > most) n = most;
+  const int64_t chunk = cdiv(cdiv(p->Tk, n), 64) * 64;
+  sp.nsplit = (int)cdiv(p->Tk, chunk);
+  sp.chunk = (int)chunk;
+  sp.unit_waves = 1;
   return sp;
 }
 
@@ -496,7 +526,7 @@ static_assert(sigattn::kSplitScratchBytes == SIGATTN_NOALLOC_SCRATCH_BYTES, "scr
 // (batch, head)).  The range split of small dense grids runs only with a
 // caller workspace.
 static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t workspace_bytes,
-                    bool static_scratch, void *stream) {
+                    bool static_scratch, void *stream, bool decode = false) {
   const int rc = sigattn_check(p);
   if (rc != SIGATTN_OK) return rc;
   const hipStream_t st = (hipStream_t)stream;
@@ -515,6 +545,10 @@ static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t
   const void *ptrs[4] = {p->q, p->k, p->v, out};
   const bool mfma = use_mfma(p, ptrs, 4);
   SplitPlan sp = splitkv_plan(p, mfma);
+  if (decode && workspace != nullptr) {
+    const SplitPlan dp = decode_plan(p, mfma);
+    if (dp.nsplit > 0) sp = dp;
+  }
   if (sp.nsplit > 1 && static_scratch) {
     if ((size_t)splitkv_workspace_bytes(p, sp) > sigattn::kSplitScratchBytes) return SIGATTN_ERR_SCRATCH;
     float *ws = nullptr;
@@ -554,6 +588,7 @@ static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t
   if (sp.nsplit > 0) {
     k.nsplit = sp.nsplit;
     k.chunk = sp.chunk;
+    k.unit_waves = sp.unit_waves;
     sigattn::launch_fwd_splitkv(k, p->dtype, (int)p->D, p->score_mod != nullptr, st);
   } else if (mfma) {
     sigattn::launch_fwd_mfma(k, p->dtype, mfma_head_dim(p), p->causal != 0, p->score_mod != nullptr, st);
@@ -568,6 +603,19 @@ static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t
 int sigattn_fwd_ws(const sigattn_problem *p, void *out, void *workspace, size_t workspace_bytes,
                    void *stream) {
   return fwd_impl(p, out, workspace, workspace_bytes, false, stream);
+}
+
+size_t sigattn_fwd_decode_workspace_bytes(const sigattn_problem *p) {
+  if (sigattn_check(p) != SIGATTN_OK || p->B == 0 || p->H == 0 || p->Tq == 0) return 0;
+  const void *none[1] = {nullptr};
+  const SplitPlan dp = decode_plan(p, use_mfma(p, none, 0));
+  if (dp.nsplit > 0) return (size_t)splitkv_workspace_bytes(p, dp);
+  return sigattn_fwd_workspace_bytes(p);
+}
+
+int sigattn_fwd_decode(const sigattn_problem *p, void *out, void *workspace, size_t workspace_bytes,
+                       void *stream) {
+  return fwd_impl(p, out, workspace, workspace_bytes, false, stream, true);
 }
 
 int sigattn_fwd(const sigattn_problem *p, void *out, void *stream) {

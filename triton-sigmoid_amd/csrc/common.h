@@ -98,7 +98,8 @@ struct KParams {
   int nblk;  // number of row blocks along the stationary sequence axis
   // Split-KV forward: keys cut into nsplit chunks of `chunk` keys; fp32
   // partials [nsplit, B, H, Tq, D] in ws when nsplit > 1.
-  int nsplit, chunk;
+  // unit_waves: waves that share one (batch, head, chunk), 4 or 1.
+  int nsplit, chunk, unit_waves;
   float *ws;
   // Two-pass backward: dS in the I/O dtype as 32x32 tiles (see DsLayout),
   // written by the dK/dV kernel and read by the dQ-from-dS kernel.
@@ -656,6 +657,8 @@ template <int ROWS, int D, int NWAVES> struct DmaPlan {
   // of any stage, which serialises the prefetch with the compute it should
   // overlap.  The kernels wait for the copy themselves (wait_dma() and a
   // barrier) before any wave reads the stage it fills.
+  // NT: non-temporal loads, for rows that are read once.
+  template <bool NT = false>
   __device__ __forceinline__ void issue(uint16_t *lds, const uint16_t *base, int stride_bytes,
                                         int row0, int nvalid) const {
 #pragma unroll
@@ -665,10 +668,16 @@ template <int ROWS, int D, int NWAVES> struct DmaPlan {
       // The low 32 bits of a generic LDS pointer are its LDS offset.
       const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds + r0[i] * D));
       // M0 holds the LDS destination; s_nop covers the M0-write -> LDS-DMA wait state.
-      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :
-                   : "v"(off), "s"(base), "{m0}"(dst)
-                   : "memory");
+      if constexpr (NT)
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                     :
+                     : "v"(off), "s"(base), "{m0}"(dst)
+                     : "memory");
+      else
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(off), "s"(base), "{m0}"(dst)
+                     : "memory");
     }
   }
 };

@@ -12,14 +12,13 @@
 // second kernel sums the partials in chunk order (deterministic).  With one
 // chunk the workgroup writes O itself and no workspace is used.
 //
-// Workgroup: four waves, 32 queries (the MFMA's 32 columns), one key chunk.
-// Wave w takes the 32-key blocks w, w+4, w+8, ... of the chunk.  Each wave
-// streams its own blocks through a private two-stage LDS ring with direct
+// Workgroup: four waves, 32 queries (the MFMA's 32 columns); the waves share
+// one key chunk or take one each (unit_waves below).  Each wave streams its
+// own 32-key blocks through a private two-stage LDS ring with direct
 // global->LDS copies and waits for them with its own vmcnt, so the key loop has
 // no workgroup barriers.  The kernel is HBM-bound (2·D·2 bytes of K and V per
 // key against 4·D·32 MFMA FLOPs), so each block is computed as a plain
-// sequence: Sᵀ = K·Qᵀ, P = sigmoid(Sᵀ) on packed words, Oᵀ += Vᵀ·Pᵀ.  The four
-// waves' Oᵀ partials are summed through LDS at the end.
+// sequence: Sᵀ = K·Qᵀ, P = sigmoid(Sᵀ) on packed words, Oᵀ += Vᵀ·Pᵀ.
 #include <atomic>
 #include <mutex>
 
@@ -74,44 +73,62 @@ hipError_t splitkv_scratch(float **ptr) {
   return hipSuccess;
 }
 
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Waits until at most `ahead` blocks of copies (PER instructions each) are in
-// flight, ahead < 4.
-template <int PER> __device__ __forceinline__ void wait_blocks(int ahead) {
-  if (ahead <= 0) wait_vmcnt<0>();
-  else if (ahead == 1) wait_vmcnt<PER>();
-  else if (ahead == 2) wait_vmcnt<2 * PER>();
-  else wait_vmcnt<3 * PER>();
-}
-
-template <typename T, int D, int NW, int NST, bool SCOREMOD, bool DIRECT>
-__global__ __launch_bounds__(64 * NW, 1) void fwd_splitkv_kernel(const KParams p) {
-  // NW waves; each streams 32-key blocks through its own NST-stage ring and
-  // keeps NST - 1 blocks of copies in flight while it computes one.
+// Two forms of the chunk kernel, by the waves that share a unit (one chunk
+// of one (batch, head)):
+//   * WPU = 4: the workgroup's waves take every fourth 32-key block of its
+//     chunk and add their partials through LDS -- short caches, where there
+//     are too few chunks to give every wave one of its own;
+//   * WPU = 1: every wave has a unit of its own, the units of one key range
+//     in head order, so the four waves of a workgroup read the rows of four
+//     neighbouring heads (4 * 2 * D contiguous bytes of every [B, T, H, D]
+//     row) and never wait for each other.  What bounds the kernel is the read
+//     of K and V, and how fast that goes follows from the contiguous bytes a
+//     workgroup reads at a time and from the loads' cache policy.  A plain
+//     read of 1 GiB by 256-byte (128-byte) rows of one head per workgroup
+//     reaches 6.0 (5.0) TB/s, non-temporal 6.4 (5.7), by four heads per
+//     workgroup and non-temporal 6.8 (6.8), and contiguous 6.8.  The calls
+//     themselves, from WPU = 4 with plain loads: bf16 B=16 H=32 D=128 Tq=1
+//     Tk=8192 493 -> 323 us (6.6 TB/s), B=1 Tk=131072 390 -> 324 us, B=32
+//     H=32 D=64 Tq=4 Tk=4096 216 -> 166 us (6.9 TB/s without the calls' other
+//     launches); one-wave workgroups on the heads of one XCD took 348, 364 and
+//     214 us, two-wave ones 317, 317 and 191.
+// A wave's K and V blocks have two stages each; the K stage is refilled as
+// soon as S is computed and the V stage after the output product, so three of
+// the four blocks are in flight at any time.
+template <typename T, int D, int WPU, bool SCOREMOD, bool DIRECT>
+__global__ __launch_bounds__(256, 1) void fwd_splitkv_kernel(const KParams p) {
+  constexpr int NW = 4;
   constexpr int KB = 32;         // keys per block (one MFMA contraction of 2 k-steps)
   constexpr int NKS = D / 16, NDB = D / 32;
-  static_assert(NST >= 2 && NST <= 4, "ring depth");
   using Plan = DmaPlan<KB, D, 1>;
-  constexpr int NI = Plan::NI;   // copy instructions per block and tensor
+  constexpr int NI = Plan::NI;   // copy instructions per block of V
+  constexpr int NK = NI + (SCOREMOD ? 1 : 0);  // ... of K, with its keys' score_mod
 
-  __shared__ __attribute__((aligned(16))) uint16_t sK[NW][NST][KB * D];
-  __shared__ __attribute__((aligned(16))) uint16_t sV[NW][NST][KB * D];
-  static_assert(sizeof(sK) >= NW * 32 * D * sizeof(float), "reduction buffer");
-
-  const int NS = p.nsplit, C = p.chunk;
-  const int s = blockIdx.x % NS, bh = blockIdx.x / NS;
-  const int b = bh / p.H, h = bh % p.H;
-  const int Lq = p.len_q(b), Lk = p.len_k(b);
-  const int k0 = s * C, k1 = min(k0 + C, Lk);
-  // A chunk past the keys has no partial (the reduction stops before it).
-  if (!DIRECT && (k0 >= Lk || Lq == 0)) return;
+  __shared__ __attribute__((aligned(16))) uint16_t sK[NW][2][KB * D];
+  __shared__ __attribute__((aligned(16))) uint16_t sV[NW][2][KB * D];
+  __shared__ __attribute__((aligned(16))) float sM[SCOREMOD ? NW : 1][2][64];
+  static_assert(WPU == 1 || sizeof(sK) >= NW * 32 * D * sizeof(float), "reduction buffer");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
+  const int NS = p.nsplit, C = p.chunk;
+  int s, b, h;
+  if (WPU == 1) {
+    const unsigned u = blockIdx.x * NW + w, H = p.H, r = u / H;  // units fit 31 bits (sigattn_check)
+    if (u >= H * (unsigned)p.B * (unsigned)NS) return;
+    h = (int)(u - r * H);
+    s = (int)(r % (unsigned)NS);
+    b = (int)(r / (unsigned)NS);
+  } else {
+    const int bh = blockIdx.x / NS;
+    s = blockIdx.x % NS, b = bh / p.H, h = bh % p.H;
+  }
+  const int wu = WPU == 1 ? 0 : w;  // the wave's place in its unit
+  const int Lq = p.len_q(b), Lk = p.len_k(b);
+  const int k0 = s * C, k1 = min(k0 + C, Lk);
+  // A chunk past the keys has no partial (the reduction stops before it).
+  if (!DIRECT && (k0 >= Lk || Lq == 0)) return;
 
   const int64_t qoff = p.q_base(b, h), koff = p.k_base(b, h);
   const uint16_t *Qb = (const uint16_t *)p.q + qoff;
@@ -130,9 +147,6 @@ __global__ __launch_bounds__(64 * NW, 1) void fwd_splitkv_kernel(const KParams p
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qf[ks] = ok ? *(const u32x4 *)(qrow + 16 * ks) : zero4();
   }
-  // Wait for Q here, before the first tile copy is in flight.
-#pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) asm volatile("" ::"v"(qf[ks]));
 
   f32x16 acc[NDB];
 #pragma unroll
@@ -143,33 +157,60 @@ __global__ __launch_bounds__(64 * NW, 1) void fwd_splitkv_kernel(const KParams p
   Plan dma;
   dma.init(0, lane);
   const int kv_stride_bytes = (int)(p.sk_t * 2);
-  const int nb = k1 > k0 ? (k1 - k0 + KB - 1) / KB : 0;   // blocks of the chunk
-  const int nbw = nb > w ? (nb - w + NW - 1) / NW : 0;    // ... of this wave
-  auto first_key = [&](int i) SIGATTN_INLINE { return k0 + KB * (w + NW * i); };
-  auto issue = [&](int st, int i) SIGATTN_INLINE {
-    dma.issue(sK[w][st], Kb, kv_stride_bytes, first_key(i), Lk);
-    dma.issue(sV[w][st], Vb, kv_stride_bytes, first_key(i), Lk);
+  const int nb = k1 > k0 ? (k1 - k0 + KB - 1) / KB : 0;     // blocks of the unit
+  const int nbw = nb > wu ? (nb - wu + WPU - 1) / WPU : 0;  // ... of this wave
+  auto first_key = [&](int i) SIGATTN_INLINE { return k0 + KB * (wu + WPU * i); };
+  const float *mod = SCOREMOD ? p.score_mod + p.mod_base(b) : nullptr;
+  auto issue_k = [&](int i) SIGATTN_INLINE {
+    dma.template issue<WPU == 1>(sK[w][i & 1], Kb, kv_stride_bytes, first_key(i), Lk);
+    if constexpr (SCOREMOD) {
+      // Keys first_key(i) + lane (the block's 32 are used; rows past Lk as in
+      // the K copy): lane l writes LDS bytes dst + 4 l.
+      const uint32_t off = 4u * (uint32_t)min(first_key(i) + lane, Lk - 1);
+      const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)sM[w][i & 1]);
+      asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(mod), "{m0}"(dst) : "memory");
+    }
+  };
+  auto issue_v = [&](int i) SIGATTN_INLINE {
+    dma.template issue<WPU == 1>(sV[w][i & 1], Vb, kv_stride_bytes, first_key(i), Lk);
   };
 
 #pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (i < nbw) issue(i, i);
-  for (int i = 0; i < nbw; ++i) {
-    const int st = i % NST;
-    // Block i + NST - 1 goes into the stage block i - 1 used; every LDS read
-    // of that block has returned (its MFMAs were issued) before the copy.
-    if (i + NST - 1 < nbw) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue((i + NST - 1) % NST, i + NST - 1);
+  for (int i = 0; i < 2; ++i)
+    if (i < nbw) {
+      issue_k(i);
+      issue_v(i);
     }
-    // Block i has landed once at most the blocks after it are in flight.
-    wait_blocks<2 * NI>(min(NST - 1, nbw - 1 - i));
-    const uint16_t *tK = sK[w][st];
-    const uint16_t *tV = sV[w][st];
+  // The wait for Q (which also waits for the copies above) stays out of the loop.
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) asm volatile("" ::"v"(qf[ks]));
+  for (int i = 0; i < nbw; ++i) {
+    // Copies in issue order: K(i) V(i) K(i+1) V(i+1) K(i+2) ...
+    if (i + 1 < nbw) wait_vm<2 * NI + NK>();
+    else wait_vm<NI>();
+    const uint16_t *tK = sK[w][i & 1];
+    const uint16_t *tV = sV[w][i & 1];
 
     f32x16 sc = zero16();
+    float c[16];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 m = {nbl, nbl, nbl, nbl};
+      if (SCOREMOD) {
+        const f32x4 x = *(const f32x4 *)&sM[w][i & 1][8 * g + 4 * hi];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m[j] = -(bias + x[j]) * kLog2e;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[4 * g + j] = m[j];
+    }
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) sc = Elem<T>::mfma(ld_row<D>(tK, to, 0, ks), qf[ks], sc);
+    if (i + 2 < nbw) {
+      // Every read of K(i) has returned before the copy that replaces it.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue_k(i + 2);
+    }
 
     // P words: accumulator element i of lane (l32, hi) is key
     // kb + 8(i/4) + 4hi + i%4 of query l32; keys at or past k1 get P = 0.
@@ -179,24 +220,49 @@ __global__ __launch_bounds__(64 * NW, 1) void fwd_splitkv_kernel(const KParams p
     for (int e = 0; e < 8; ++e) {
       const int i0 = 2 * e;
       const int key = kb + 8 * (i0 / 4) + 4 * hi + (i0 % 4);
-      float c0 = nbl, c1 = nbl;
-      if (SCOREMOD) {
-        const int64_t mb = p.mod_base(b);
-        c0 = key < k1 ? -(bias + p.score_mod[mb + key]) * kLog2e : 0.0f;
-        c1 = key + 1 < k1 ? -(bias + p.score_mod[mb + key + 1]) * kLog2e : 0.0f;
-      }
-      float p0 = sigmoid_from_neg_log2(__builtin_fmaf(sc[i0], nsl, c0));
-      float p1 = sigmoid_from_neg_log2(__builtin_fmaf(sc[i0 + 1], nsl, c1));
+      float p0 = sigmoid_from_neg_log2(__builtin_fmaf(sc[i0], nsl, c[i0]));
+      float p1 = sigmoid_from_neg_log2(__builtin_fmaf(sc[i0 + 1], nsl, c[i0 + 1]));
       p0 = key < k1 ? p0 : 0.0f;
       p1 = key + 1 < k1 ? p1 : 0.0f;
       pk[e] = Elem<T>::pack(p0, p1);
     }
+    if (i + 2 < nbw) wait_vm<NI + 2 * NK>();
+    else if (i + 1 < nbw) wait_vm<NI + NK>();
+    else wait_vm<0>();
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const u32x4 bp = (u32x4){pk[4 * j], pk[4 * j + 1], pk[4 * j + 2], pk[4 * j + 3]};
 #pragma unroll
       for (int db = 0; db < NDB; ++db) acc[db] = Elem<T>::mfma(ld_tr<D>(tV, to, j, db), bp, acc[db]);
     }
+    if (i + 2 < nbw) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue_v(i + 2);
+    }
+  }
+
+  float *ws_row = nullptr;
+  if (!DIRECT) ws_row = p.ws + (((int64_t)s * p.B + b) * p.H + h) * p.Tq * D;
+  uint16_t *Ob = (uint16_t *)p.out + qoff;
+  if constexpr (WPU == 1) {
+    const bool valid = l32 < Lq;
+    if (l32 < (DIRECT ? min(32, p.q_rows_out(Lq)) : min(32, Lq))) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int d0 = db * 32 + 8 * g + 4 * hi;
+          const f32x4 v = {acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+          if (DIRECT) {
+            u32x2 o = {Elem<T>::pack(v.x, v.y), Elem<T>::pack(v.z, v.w)};
+            if (!valid) o = (u32x2){0u, 0u};
+            *(u32x2 *)(Ob + (int64_t)l32 * p.sq_t + d0) = o;
+          } else {
+            *(f32x4 *)(ws_row + l32 * D + d0) = v;
+          }
+        }
+    }
+    return;
   }
 
   // Sum the waves' Oᵀ partials: red[w][q][d] in the tile memory.
@@ -225,68 +291,63 @@ __global__ __launch_bounds__(64 * NW, 1) void fwd_splitkv_kernel(const KParams p
       o.x = Elem<T>::pack(v.x, v.y);
       o.y = Elem<T>::pack(v.z, v.w);
       if (q >= Lq) o = (u32x2){0u, 0u};
-      *(u32x2 *)((uint16_t *)p.out + qoff + (int64_t)q * p.sq_t + d0) = o;
+      *(u32x2 *)(Ob + (int64_t)q * p.sq_t + d0) = o;
     } else {
-      float *ws = p.ws + ((((int64_t)s * p.B + b) * p.H + h) * p.Tq + q) * D;
-      *(float4 *)&ws[d0] = v;
+      *(float4 *)&ws_row[q * D + d0] = v;
     }
   }
 }
 
-// O = sum of the chunks' partials, in chunk order; padded query rows are zero.
+// O = sum of the chunks' partials; padded query rows are zero.  One output
+// row per workgroup: 256 / (D/4) thread groups each add every NG-th chunk's
+// partial in chunk order, and the groups' sums are added in group order, so
+// the sum is deterministic and its chain of loads NG times shorter than one
+// thread's over all chunks.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void fwd_splitkv_reduce_kernel(const KParams p) {
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t total = (int64_t)p.B * p.H * p.Tq * (D / 4);
-  if (t >= total) return;
-  const int d0 = 4 * (int)(t % (D / 4));
-  const int64_t r = t / (D / 4);
-  const int q = (int)(r % p.Tq);
-  const int bh = (int)(r / p.Tq), b = bh / p.H, h = bh % p.H;
+  constexpr int CG = D / 4, NG = 256 / CG;
+  __shared__ f32x4 part[NG][CG];
+  const int c = threadIdx.x % CG, g = threadIdx.x / CG;
+  const int q = (int)(blockIdx.x % p.Tq);
+  const int bh = (int)(blockIdx.x / p.Tq), b = bh / p.H, h = bh % p.H;
   const int Lq = p.len_q(b), Lk = p.len_k(b);
   if (q >= p.q_rows_out(Lq)) return;
-  float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
   if (q < Lq) {
     const int nvs = (Lk + p.chunk - 1) / p.chunk;
-    for (int s = 0; s < nvs; ++s) {
-      const float4 u = *(const float4 *)&p.ws[((((int64_t)s * p.B + b) * p.H + h) * p.Tq + q) * D + d0];
-      v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
-    }
+    const int64_t step = (int64_t)p.B * p.H * p.Tq * D;
+    const float *src = p.ws + ((int64_t)bh * p.Tq + q) * D + 4 * c;
+#pragma unroll 4
+    for (int s = g; s < nvs; s += NG) v += *(const f32x4 *)(src + s * step);
   }
-  u32x2 o;
-  o.x = Elem<T>::pack(v.x, v.y);
-  o.y = Elem<T>::pack(v.z, v.w);
-  *(u32x2 *)((uint16_t *)p.out + p.q_base(b, h) + (int64_t)q * p.sq_t + d0) = o;
+  part[g][c] = v;
+  __syncthreads();
+  if (g != 0) return;
+#pragma unroll
+  for (int x = 1; x < NG; ++x) v += part[x][c];
+  const u32x2 o = {Elem<T>::pack(v.x, v.y), Elem<T>::pack(v.z, v.w)};
+  *(u32x2 *)((uint16_t *)p.out + p.q_base(b, h) + (int64_t)q * p.sq_t + 4 * c) = o;
 }
 
-#ifndef SIGATTN_DEC_NW_64
-#define SIGATTN_DEC_NW_64 4
-#endif
-#ifndef SIGATTN_DEC_NST_64
-#define SIGATTN_DEC_NST_64 2
-#endif
-#ifndef SIGATTN_DEC_NW_128
-#define SIGATTN_DEC_NW_128 4
-#endif
-#ifndef SIGATTN_DEC_NST_128
-#define SIGATTN_DEC_NST_128 2
-#endif
+template <typename T, int D, int WPU>
+static void launch_chunks(const KParams &p, bool scoremod, hipStream_t st) {
+  const int64_t units = (int64_t)p.B * p.H * p.nsplit;
+  const dim3 grid((unsigned)(WPU == 1 ? (units + 3) / 4 : units)), block(256);
+  if (p.nsplit == 1) {
+    if (scoremod) fwd_splitkv_kernel<T, D, WPU, true, true><<<grid, block, 0, st>>>(p);
+    else fwd_splitkv_kernel<T, D, WPU, false, true><<<grid, block, 0, st>>>(p);
+  } else {
+    if (scoremod) fwd_splitkv_kernel<T, D, WPU, true, false><<<grid, block, 0, st>>>(p);
+    else fwd_splitkv_kernel<T, D, WPU, false, false><<<grid, block, 0, st>>>(p);
+  }
+}
 
 template <typename T, int D>
 static void launch_splitkv_t(const KParams &p, bool scoremod, hipStream_t st) {
-  constexpr int NW = D == 64 ? SIGATTN_DEC_NW_64 : SIGATTN_DEC_NW_128;
-  constexpr int NST = D == 64 ? SIGATTN_DEC_NST_64 : SIGATTN_DEC_NST_128;
-  const dim3 grid((unsigned)((int64_t)p.B * p.H * p.nsplit)), block(64 * NW);
-  const bool direct = p.nsplit == 1;
-  if (direct) {
-    if (scoremod) fwd_splitkv_kernel<T, D, NW, NST, true, true><<<grid, block, 0, st>>>(p);
-    else fwd_splitkv_kernel<T, D, NW, NST, false, true><<<grid, block, 0, st>>>(p);
-    return;
-  }
-  if (scoremod) fwd_splitkv_kernel<T, D, NW, NST, true, false><<<grid, block, 0, st>>>(p);
-  else fwd_splitkv_kernel<T, D, NW, NST, false, false><<<grid, block, 0, st>>>(p);
-  const int64_t total = (int64_t)p.B * p.H * p.Tq * (D / 4);
-  fwd_splitkv_reduce_kernel<T, D><<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st>>>(p);
+  if (p.unit_waves == 1) launch_chunks<T, D, 1>(p, scoremod, st);
+  else launch_chunks<T, D, 4>(p, scoremod, st);
+  if (p.nsplit > 1)
+    fwd_splitkv_reduce_kernel<T, D><<<dim3((unsigned)((int64_t)p.B * p.H * p.Tq)), dim3(256), 0, st>>>(p);
 }
 
 void launch_fwd_splitkv(const KParams &p, int dtype, int D, bool scoremod, hipStream_t st) {

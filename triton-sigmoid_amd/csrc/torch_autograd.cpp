@@ -11,8 +11,8 @@
 // launches the library's forward on the canonical tensors the Python layer
 // prepared and saves them; the backward launches the library's backward on
 // them.  Launch policy is the Python layer's (_capi._launch_fwd,
-// _capi._launch_bwd): the forward passes the workspace
-// sigattn_fwd_workspace_bytes asks for; the backward takes the range-split
+// _capi._launch_bwd): the forward is sigattn_fwd_decode with the workspace it
+// asks for; the backward takes the range-split
 // recompute backward when a small grid splits, else the two-pass kernels at
 // the head dims and workspace limit the Python layer configures (in head
 // groups when the whole problem's dS does not fit, unless a group's
@@ -47,6 +47,8 @@ struct Api {
   decltype(&sigattn_strerror) strerror = nullptr;
   decltype(&sigattn_fwd_workspace_bytes) fwd_workspace_bytes = nullptr;
   decltype(&sigattn_fwd_ws) fwd_ws = nullptr;
+  decltype(&sigattn_fwd_decode_workspace_bytes) fwd_decode_workspace_bytes = nullptr;
+  decltype(&sigattn_fwd_decode) fwd_decode = nullptr;
   decltype(&sigattn_bwd_workspace_bytes) bwd_workspace_bytes = nullptr;
   decltype(&sigattn_bwd_ws) bwd_ws = nullptr;
   decltype(&sigattn_bwd_split_workspace_bytes) bwd_split_workspace_bytes = nullptr;
@@ -187,8 +189,15 @@ struct SigattnNode : public torch::autograd::Function<SigattnNode> {
     const c10::DeviceGuard guard(q.device());
     const sigattn_problem p = make_problem(q, k, v, bias, sm, scale, lay, causal);
     const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
-    const int64_t nbytes = (int64_t)g_api.fwd_workspace_bytes(&p);
-    Tensor ws = nbytes > 0 ? at::empty({nbytes}, q.options().dtype(at::kByte)) : Tensor();
+    int64_t nbytes = (int64_t)g_api.fwd_decode_workspace_bytes(&p);
+    Tensor ws = workspace(nbytes, q);
+    if (nbytes == 0 || ws.defined()) {
+      check_rc(g_api.fwd_decode(&p, out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr, nbytes, stream),
+               "sigattn_fwd");
+      return out;
+    }
+    nbytes = (int64_t)g_api.fwd_workspace_bytes(&p);
+    if (nbytes > 0) ws = at::empty({nbytes}, q.options().dtype(at::kByte));
     check_rc(g_api.fwd_ws(&p, out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr, nbytes, stream),
              "sigattn_fwd");
     return out;
@@ -257,6 +266,8 @@ void bind(const py::dict &fns, const std::vector<int64_t> &two_pass_dims, int64_
   bind_one(api.strerror, fns, "sigattn_strerror");
   bind_one(api.fwd_workspace_bytes, fns, "sigattn_fwd_workspace_bytes");
   bind_one(api.fwd_ws, fns, "sigattn_fwd_ws");
+  bind_one(api.fwd_decode_workspace_bytes, fns, "sigattn_fwd_decode_workspace_bytes");
+  bind_one(api.fwd_decode, fns, "sigattn_fwd_decode");
   bind_one(api.bwd_workspace_bytes, fns, "sigattn_bwd_workspace_bytes");
   bind_one(api.bwd_ws, fns, "sigattn_bwd_ws");
   bind_one(api.bwd_split_workspace_bytes, fns, "sigattn_bwd_split_workspace_bytes");

@@ -70,6 +70,8 @@ SIGNATURES = {
     "sigattn_fwd": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp], _c_i32),
     "sigattn_fwd_workspace_bytes": ([ctypes.POINTER(SigattnProblem)], ctypes.c_size_t),
     "sigattn_fwd_ws": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp, ctypes.c_size_t, _c_vp], _c_i32),
+    "sigattn_fwd_decode_workspace_bytes": ([ctypes.POINTER(SigattnProblem)], ctypes.c_size_t),
+    "sigattn_fwd_decode": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp, ctypes.c_size_t, _c_vp], _c_i32),
     "sigattn_fwd_noalloc": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp], _c_i32),
     "sigattn_bwd": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp, _c_vp, _c_vp, _c_vp], _c_i32),
     "sigattn_bwd_dq": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp, _c_vp], _c_i32),
@@ -127,6 +129,7 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
 # so does a node that fails to import (with a warning).
 _EAGER_ENV = "SIGATTN_EAGER_BINDING"
 _AUTOGRAD_FNS = ("sigattn_strerror", "sigattn_fwd_workspace_bytes", "sigattn_fwd_ws",
+                 "sigattn_fwd_decode_workspace_bytes", "sigattn_fwd_decode",
                  "sigattn_bwd_workspace_bytes", "sigattn_bwd_ws", "sigattn_bwd_split_workspace_bytes",
                  "sigattn_bwd_split")
 _autograd = None  # the bound module, or False after a failed import
@@ -266,10 +269,16 @@ def _on_device(dev: torch.device, fn):
 
 
 def _launch_fwd(lib, pr: SigattnProblem, out: torch.Tensor) -> None:
-    """sigattn_fwd_ws with the workspace the problem asks for (decode shapes
-    split their keys over several workgroups; others need none), allocated
-    from torch's caching allocator on the output's device."""
+    """sigattn_fwd_decode with the workspace the problem asks for (decode
+    shapes and small grids split their keys over several workgroups; others
+    need none), allocated from torch's caching allocator on the output's
+    device; sigattn_fwd_ws and its smaller one when that does not fit."""
     def run(stream):
+        nbytes = int(lib.sigattn_fwd_decode_workspace_bytes(ctypes.byref(pr)))
+        ws, got = _bwd_workspace(nbytes, out.device)
+        if got == nbytes:
+            _raise(lib.sigattn_fwd_decode(ctypes.byref(pr), out.data_ptr(), _ptr(ws), nbytes, stream), "sigattn_fwd")
+            return
         nbytes = int(lib.sigattn_fwd_workspace_bytes(ctypes.byref(pr)))
         ws = torch.empty(nbytes, dtype=torch.uint8, device=out.device) if nbytes else None
         _raise(lib.sigattn_fwd_ws(ctypes.byref(pr), out.data_ptr(), _ptr(ws), nbytes, stream), "sigattn_fwd")
@@ -337,10 +346,10 @@ def bwd_workspace_bytes(lib, pr: SigattnProblem, device: torch.device) -> int:
 
 
 def _bwd_workspace(nbytes: int, device: torch.device):
-    """The two-pass backward's dS workspace, or None when it is not used or
-    the device cannot hold it: the recompute backward needs no workspace, so
-    an allocation failure falls back to it instead of failing the backward
-    (the reference's backward allocates only its outputs)."""
+    """A workspace that the call can do without (the two-pass backward's dS,
+    a forward's partials), or None when it is not used or the device cannot
+    hold it: the kernels that need none, or less, then run instead of the call
+    failing (the reference allocates only its outputs)."""
     if nbytes == 0:
         return None, 0
     try:
