@@ -103,6 +103,15 @@ const char *sigattn_strerror(int status);
 int sigattn_check(const sigattn_problem *p);
 
 /*
+ * The default bias of ragged batches, bias[b] = -log(n) in fp32 with n the key
+ * length of sequence b (sigmoid_triton_padded.py:995-996): seq_lens[b], or
+ * cu_seqlens[b + 1] - cu_seqlens[b]; exactly one of the two is given.  One
+ * kernel on `stream`.
+ */
+int sigattn_default_bias(const int32_t *seq_lens, const int32_t *cu_seqlens, int64_t B, float *bias,
+                         void *stream);
+
+/*
  * Forward: out[B, Tq, H, D] (q strides).  Rows at or past seq_lens_q[b] are
  * written as zeros (packed layout: rows outside every sequence are zeros).
  * `stream` is a hipStream_t (NULL = default stream).

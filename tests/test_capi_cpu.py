@@ -329,3 +329,13 @@ def test_device_constants_are_never_freed(monkeypatch):
     assert isinstance(extra, torch.Tensor) and len(_capi._CONSTANTS) == 3
     assert all(_capi._CONSTANTS[((2,), float(i), torch.float32, torch.device("cuda", 0))] is first[i]
                for i in range(3))
+
+
+def test_default_bias_errors():
+    lib = _capi.load_library()
+    fake = 1 << 20
+    assert lib.sigattn_default_bias(fake, None, -1, fake, None) == -4
+    assert lib.sigattn_default_bias(None, None, 0, None, None) == 0
+    assert lib.sigattn_default_bias(fake, None, 2, None, None) == -1
+    assert lib.sigattn_default_bias(None, None, 2, fake, None) == -1
+    assert lib.sigattn_default_bias(fake, fake, 2, fake, None) == -9

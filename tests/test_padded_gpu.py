@@ -406,3 +406,20 @@ def test_concurrent_backward_equals_the_two_kernels(layout):
     if layout == "padded":
         for t in one:
             assert torch.all(t[1, 2731:] == 0)
+
+
+@pytest.mark.parametrize("B", [1, 255, 256, 257, 1000])
+def test_default_bias_kernel_equals_the_operators(B):
+    """sigattn_default_bias against -torch.log of the lengths, bit for bit:
+    lengths and packed offsets, zero, negative and huge ones, int64 input."""
+    g = torch.Generator().manual_seed(B)
+    lens = torch.randint(0, 20000, (B,), generator=g, dtype=torch.int32)
+    lens[::7] = torch.tensor([0, 1, -3, 2 ** 31 - 1, 2 ** 24 + 1], dtype=torch.int32).repeat(B)[:len(lens[::7])]
+    cu = torch.cat([torch.zeros(1, dtype=torch.int32), lens.clamp(0, 20000).cumsum(0).to(torch.int32)])
+    lens, cu = lens.to("cuda"), cu.to("cuda")
+    dev = lens.device
+    for got, n in ((_capi.default_bias(dev, seq_lens=lens), lens),
+                   (_capi.default_bias(dev, seq_lens=lens.long()), lens),
+                   (_capi.default_bias(dev, cu_seqlens=cu), cu[1:] - cu[:-1])):
+        want = -torch.log(n.to(torch.float32))
+        assert got.shape == (B,) and torch.equal(got.view(torch.int32), want.view(torch.int32))

@@ -26,7 +26,8 @@ INCLUDE = ROOT.parent / "include"
 LIB_PATH = PKG_DIR / "libsigattn.so"
 BUILD_DIR = ROOT / "_build"
 
-SOURCES = ["fwd.hip", "bwd.hip", "decode.hip", "f32.hip", "generic.hip", "capi.cpp"]
+SOURCES = ["fwd.hip", "bwd.hip", "decode.hip", "f32.hip", "generic.hip", "bias.hip", "capi.cpp"]
+SOURCE_FLAGS = {"bias.hip": ["-ffp-contract=off"]}  # see the file
 ARCH = "gfx950"
 AUTOGRAD_SOURCE = "torch_autograd.cpp"
 AUTOGRAD_NAME = "_sigattn_autograd"
@@ -53,7 +54,7 @@ def compile_flags() -> list[str]:
 
 def _compile(src: Path, obj: Path, defines: tuple = ()) -> None:
     lang = ["-x", "hip"] if src.suffix == ".cpp" else []
-    cmd = [hipcc(), *compile_flags(), *defines, *lang, "-c", str(src), "-o", str(obj)]
+    cmd = [hipcc(), *compile_flags(), *SOURCE_FLAGS.get(src.name, []), *defines, *lang, "-c", str(src), "-o", str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{res.stdout}\n{res.stderr}")

@@ -67,6 +67,7 @@ SIGNATURES = {
     "sigattn_abi_version": ([], _c_i32),
     "sigattn_strerror": ([_c_i32], ctypes.c_char_p),
     "sigattn_check": ([ctypes.POINTER(SigattnProblem)], _c_i32),
+    "sigattn_default_bias": ([_c_vp, _c_vp, _c_i64, _c_vp, _c_vp], _c_i32),
     "sigattn_fwd": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp], _c_i32),
     "sigattn_fwd_workspace_bytes": ([ctypes.POINTER(SigattnProblem)], ctypes.c_size_t),
     "sigattn_fwd_ws": ([ctypes.POINTER(SigattnProblem), _c_vp, _c_vp, ctypes.c_size_t, _c_vp], _c_i32),
@@ -515,6 +516,27 @@ def backward_packed(Q, K, V, dO, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_s
                   packed=_packed_dims(Q, K, cu_q, cu_k, max_seqlen_q, max_seqlen_k))
     _launch_bwd(lib, pr, dO, dQ, dK, dV)
     return dQ, dK, dV
+
+
+def default_bias(device: torch.device, seq_lens: Optional[torch.Tensor] = None,
+                 cu_seqlens: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """-log(key length) per sequence, [B] fp32 on `device`, from int32 lengths
+    [B] or offsets [B + 1].  Eagerly on a GPU one kernel; under torch.compile
+    and for CPU tensors (which the ops then refuse) element-wise operators
+    with the same results."""
+    src = seq_lens if seq_lens is not None else cu_seqlens
+    if torch.compiler.is_compiling() or device.type != "cuda" or type(src) is not torch.Tensor:
+        n = seq_lens if seq_lens is not None else cu_seqlens[1:] - cu_seqlens[:-1]
+        return -torch.log(n.to(device=device, dtype=torch.float32))
+    src = _as(src, torch.int32, device)
+    B = src.numel() - (seq_lens is None)
+    bias = torch.empty((B,), dtype=torch.float32, device=device)
+    lib = load_library()
+    _check_device(bias)
+    _on_device(bias.device, lambda stream: _raise(lib.sigattn_default_bias(
+        src.data_ptr() if seq_lens is not None else None, src.data_ptr() if seq_lens is None else None, B,
+        bias.data_ptr(), stream), "sigattn_default_bias"))
+    return bias
 
 
 _CONSTANTS: dict = {}

@@ -191,7 +191,7 @@ def sigmoid_attention_padded(
 
     # Default bias -log(seq_lens_k) with no epsilon (sigmoid_triton_padded.py:995-996).
     if sigmoid_bias is None:
-        bias = -torch.log(seq_lens_k.to(device=query.device, dtype=torch.float32))
+        bias = _capi.default_bias(query.device, seq_lens=seq_lens_k)
     else:
         bias = _capi.device_constant((B,), float(sigmoid_bias), torch.float32, query.device)
 

@@ -205,11 +205,10 @@ def sigmoid_attention_varlen(
             raise ValueError(f"score_mod must have shape ({N_k},), got {score_mod.shape}")
         score_mod = score_mod.contiguous()
 
-    lens_k = (cu_seqlens_k[1:] - cu_seqlens_k[:-1]).to(device=query.device)
     if max_seqlen_q is None:
         max_seqlen_q = int((cu_seqlens_q[1:] - cu_seqlens_q[:-1]).max().item()) if B > 0 else 0
     if max_seqlen_k is None:
-        max_seqlen_k = int(lens_k.max().item()) if B > 0 else 0
+        max_seqlen_k = int((cu_seqlens_k[1:] - cu_seqlens_k[:-1]).max().item()) if B > 0 else 0
     if max_seqlen_q < 0 or max_seqlen_k < 0:
         raise ValueError(f"max_seqlen must be non-negative, got q={max_seqlen_q}, k={max_seqlen_k}")
 
@@ -220,7 +219,7 @@ def sigmoid_attention_varlen(
             torch._dynamo.mark_static(x, -1)
 
     if sigmoid_bias is None:
-        bias = -torch.log(lens_k.to(torch.float32))
+        bias = _capi.default_bias(query.device, cu_seqlens=cu_seqlens_k)
     else:
         bias = _capi.device_constant((B,), float(sigmoid_bias), torch.float32, query.device)
     if scale is None:
