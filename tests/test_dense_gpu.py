@@ -403,3 +403,84 @@ def test_tiny_sequence_lengths(T):
     want, _ = oracle_fwd_bwd(q, k, v, do, scale=np.float32(1 / math.sqrt(D)),
                              bias=np.full(B, np.float32(-math.log(T))), causal=True, with_bwd=False)
     assert_close_to_oracle(o, want, torch.float16, "O")
+
+
+# --- fp32 kernels: waves per row group, and values the bf16 splits cannot hold ---
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("B,H,T", [(2, 3, 61), (2, 3, 257),      # four waves share 32 rows (two at D = 128)
+                                   (4, 17, 161),                 # two waves share 64 rows: more than 256 blocks of 32
+                                   (15, 18, 129)])               # one wave per 32 rows: 540 blocks of 128
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("with_mod", [False, True])
+def test_fp32_waves_per_rows_match_oracle(B, H, T, D, causal, with_mod):
+    """Each form of the fp32 kernels at remainders of its row blocks and
+    streamed steps, padded lengths among them, on a few of the heads."""
+    dtype = torch.float32
+    q, k, v, do = _inputs(B, T, H, D, dtype, seed=B * T + D)
+    g = torch.Generator().manual_seed(T)
+    mod = torch.randn((B, T), generator=g).to(DEV) if with_mod else None
+    lens = torch.randint(1, T + 1, (B,), generator=g, dtype=torch.int32)
+    lens[0], lens[1] = T, max(1, T - 33)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    ld = lens.to(DEV)
+    o = ts.sigmoid_attention_padded(q, k, v, ld, ld, is_causal=causal, sigmoid_bias=-2.0, score_mod=mod)
+    o.backward(do)
+    for b, h in ((0, 0), (0, H - 1), (1, 1), (B - 1, H // 2)):
+        n = int(lens[b])
+        one = [t.detach()[b:b + 1, :n, h:h + 1] for t in (q, k, v, do)]
+        want_o, grads = oracle_fwd_bwd(*one, scale=np.float32(1.0 / math.sqrt(D)), bias=np.full(1, -2.0),
+                                       causal=causal, score_mod=None if mod is None else mod[b:b + 1, :n])
+        for name, got, want in zip(("O", "dQ", "dK", "dV"), (o, q.grad, k.grad, v.grad), (want_o, *grads)):
+            assert_close_to_oracle(got[b:b + 1, :n, h:h + 1], want, dtype, name)
+            assert torch.all(got[b, n:] == 0)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])  # 16 runs at width 32, where an infinity meets zeros
+@pytest.mark.parametrize("T", [96, 320])  # whole tiles: a tail repeats the last row, and 0 * inf is NaN
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kind", ["nan", "inf", "-inf", "max", "tiny", "mask"])
+def test_fp32_values_outside_the_split_match_the_portable_kernels(D, T, causal, kind):
+    """Infinities, NaN, magnitudes above bf16's largest and below its smallest,
+    and score_mod of the type's lowest value: the fp32 kernels against the
+    portable ones (rows off 16-byte boundaries), which use plain FMAs."""
+    B, H = 2, 3
+    q, k, v, do = _inputs(B, T, H, D, torch.float32, seed=T + D)
+    mod = torch.zeros((B, T), device=DEV)
+    if kind == "tiny":
+        v.mul_(1e-36)
+        do.mul_(1e-36)
+    elif kind == "mask":
+        mod[:, T // 2:] = torch.finfo(torch.float32).min
+        mod[1, 3] = float("-inf")
+    else:
+        x = float(kind) if kind != "max" else 3.4e38
+        # The first key and the last query: no mask stands between them and any
+        # other row (a masked pair's 0 * inf is NaN in whichever kernel's tile has it).
+        q[0, T - 1, 0, 1] = x
+        k[0, 0, 1, 2] = x
+        v[1, 0, 1, 3] = x
+        do[1, T - 1, 2, 0] = x
+    lib = _capi.load_library()
+    bias = torch.full((B,), -2.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(pad):
+        # pad = 1: heads D + 1 floats apart, so most rows start off 16 bytes.
+        ins = [torch.nn.functional.pad(t, (0, pad))[..., :D] for t in (q, k, v, do)]
+        outs = [torch.nn.functional.pad(torch.full_like(t, 7.0), (0, pad))[..., :D] for t in (q, q, k, k)]
+        pr = _capi._problem(*ins[:3], bias, mod, scale, None, None, causal)
+        assert lib.sigattn_fwd(ctypes.byref(pr), outs[0].data_ptr(), stream) == 0
+        assert lib.sigattn_bwd(ctypes.byref(pr), ins[3].data_ptr(), *(t.data_ptr() for t in outs[1:]), stream) == 0
+        torch.cuda.synchronize()
+        return outs
+
+    for name, got, want in zip(("O", "dQ", "dK", "dV"), run(0), run(1)):
+        assert torch.equal(torch.isnan(got), torch.isnan(want)), name
+        assert torch.equal(torch.isinf(got), torch.isinf(want)), name
+        fine = torch.isfinite(want)
+        # fp32 sums of up to T and D terms in two orders: a few roundings of the largest value.
+        top = want[fine].abs().max().item() if fine.any() else 0.0
+        torch.testing.assert_close(got[fine], want[fine], rtol=0, atol=2 ** -24 * 64 * top)
