@@ -484,3 +484,45 @@ def test_fp32_values_outside_the_split_match_the_portable_kernels(D, T, causal, 
         # fp32 sums of up to T and D terms in two orders: a few roundings of the largest value.
         top = want[fine].abs().max().item() if fine.any() else 0.0
         torch.testing.assert_close(got[fine], want[fine], rtol=0, atol=2 ** -24 * 64 * top)
+
+
+# --- D <= 64 forward and dQ: two waves per 32 rows on small grids, one on large ones ---
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("T", [63, 65, 96, 129])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("layout", ["dense", "mod", "padded"])
+def test_wave_pairs_and_single_waves_match_oracle(D, T, causal, layout):
+    """17 x 64 (batch, head) pairs are more than four blocks per compute unit
+    (a wave per 32 rows in every kernel); one pair alone is a small grid (two
+    waves per 32 rows).  Both against the oracle, on remainders of 32-, 64-
+    and 128-row blocks."""
+    B, H, dtype = 17, 64, torch.bfloat16
+    q, k, v, do = _inputs(B, T, H, D, dtype, seed=T + D)
+    g = torch.Generator().manual_seed(T)
+    mod = torch.randn((B, T), generator=g).to(DEV) if layout == "mod" else None
+    lens = torch.full((B,), T, dtype=torch.int32)
+    if layout == "padded":
+        lens[1:] = torch.randint(1, T + 1, (B - 1,), generator=g, dtype=torch.int32)
+
+    def run(bs, hs):
+        ins = [t[bs, :, hs].contiguous().requires_grad_(True) for t in (q, k, v)]
+        m = None if mod is None else mod[bs].contiguous()
+        if layout == "padded":
+            n = lens[bs].to(DEV)
+            o = ts.sigmoid_attention_padded(*ins, n, n, is_causal=causal, sigmoid_bias=-2.0)
+        else:
+            o = ts.sigmoid_attention(*ins, is_causal=causal, sigmoid_bias=-2.0, score_mod=m)
+        return (o, *torch.autograd.grad(o, ins, do[bs, :, hs].contiguous()))
+
+    whole = run(slice(0, B), slice(0, H))
+    for b, h in ((0, 0), (3, H - 1), (B - 1, 17)):
+        n = int(lens[b])
+        alone = run(slice(b, b + 1), slice(h, h + 1))
+        one = [t[b:b + 1, :n, h:h + 1] for t in (q, k, v, do)]
+        want_o, grads = oracle_fwd_bwd(*one, scale=np.float32(1.0 / math.sqrt(D)), bias=np.full(1, -2.0),
+                                       causal=causal, score_mod=None if mod is None else mod[b:b + 1])
+        for name, x, y, want in zip(("O", "dQ", "dK", "dV"), whole, alone, (want_o, *grads)):
+            assert_close_to_oracle(x[b:b + 1, :n, h:h + 1], want, dtype, f"{name}, large grid")
+            assert_close_to_oracle(y[:, :n], want, dtype, f"{name}, alone")
+            assert torch.all(x[b, n:] == 0) and torch.all(y[:, n:] == 0)

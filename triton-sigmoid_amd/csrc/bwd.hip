@@ -32,18 +32,24 @@ namespace sigattn {
 //   dQᵀ += Kᵀ·dSᵀ with dSᵀ taken from the accumulator registers and Kᵀ read
 //   from the K tile with ds_read_b64_tr_b16.
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool CAUSAL, bool SCOREMOD>
-__device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
-  constexpr int BM = 128, BN = 64;
+// WK = 2: two pairs of waves of 32 queries; the waves of a pair hold the same
+// queries, take one 32-key block of every tile each, and their accumulators
+// are added at the end (launch_bwd_dq_mfma says where).
+template <int D, bool SCOREMOD> struct DqLds {
+  uint16_t k[2][64 * D], v[2][64 * D];
+  float c[SCOREMOD ? 2 * 64 : 4];
+};
+template <typename T, int D, int WK, bool CAUSAL, bool SCOREMOD>
+__device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg, DqLds<D, SCOREMOD> &lds) {
+  constexpr int NG = 4 / WK, BM = 32 * NG, BN = 64;
   constexpr int NKS = D / 16, NDB = D / 32;
-
-  __shared__ __attribute__((aligned(16))) uint16_t sK[2][BN * D];
-  __shared__ __attribute__((aligned(16))) uint16_t sV[2][BN * D];
-  __shared__ __attribute__((aligned(16))) float sC[SCOREMOD ? 2 * BN : 4];
+  auto &sK = lds.k;
+  auto &sV = lds.v;
+  auto &sC = lds.c;
 
   int b, h, qb;
   int ritem = 0, rchunk = 0;  // range split: the item and this workgroup's chunk of its keys
-  if (!CAUSAL && p.rsplit > 1) {
+  if (WK == 1 && !CAUSAL && p.rsplit > 1) {
     int bh;
     ritem = wg / p.rsplit, rchunk = wg % p.rsplit;
     dense_item(ritem, p.B * p.H, p.nblk, true, bh, qb);
@@ -66,7 +72,7 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
   // Keys of this workgroup: under the range split, its chunk of the item's
   // key tiles, indexed from the chunk's first key.
   int key0 = 0, Lk = p.len_k(b);
-  if (!CAUSAL && p.rsplit > 1) {
+  if (WK == 1 && !CAUSAL && p.rsplit > 1) {
     const int ntk = (Lk + BN - 1) / BN;
     key0 = split_tile(rchunk, p.rsplit, ntk) * BN;
     Lk = min(Lk, split_tile(rchunk + 1, p.rsplit, ntk) * BN) - key0;
@@ -79,9 +85,11 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
     return;
   }
 
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = WK == 2 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int l32 = lane & 31, hi = lane >> 5;
-  const int q0 = qb * BM, qw = q0 + w * 32, my_q = qw + l32;
+  const int wt = w / NG;  // place in the wave's pair (WK = 2)
+  const int q0 = qb * BM, qw = q0 + (w % NG) * 32, my_q = qw + l32;
 
   const int64_t qoff = p.q_base(b, h);
   const int64_t koff = p.k_base(b, h) + (int64_t)key0 * p.sk_t;
@@ -118,6 +126,7 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
 
   TileOffsets<D> to;
   to.init(lane);
+  if constexpr (WK == 2) to.advance(32 * wt);  // this wave's half of every tile
   DmaPlan<BN, D, 4> dma;
   dma.init(w, lane, half);
   const int kv_stride_bytes = (int)(p.sk_t * 2);
@@ -170,8 +179,9 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
   // and dO operands would not fit next to the dQ accumulators); the second
   // wave on each SIMD supplies the MFMA/VALU overlap.
   auto tile_step = [&](int st, int n0, bool mask) SIGATTN_INLINE {
+    const int cl = WK == 2 ? 32 * wt : 0;
 #pragma unroll
-    for (int kbi = 0; kbi < 2; ++kbi) {
+    for (int kbi = 0; kbi < 2 / WK; ++kbi) {
       f32x16 s = zero16(), dp = zero16();
       uint32_t dk[8];
 #pragma unroll
@@ -179,7 +189,7 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
         s = Elem<T>::mfma(ld_row<D>(sK[st], to, 32 * kbi, ks), qf[ks], s);
         dp = Elem<T>::mfma(ld_row<D>(sV[st], to, 32 * kbi, ks), of[ks], dp);
       }
-      ds_block(s, dp, st, 32 * kbi, n0 + 32 * kbi, dk, mask);
+      ds_block(s, dp, st, 32 * kbi + cl, n0 + 32 * kbi + cl, dk, mask);
       dq_block(st, kbi, dk);
     }
   };
@@ -205,7 +215,7 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
       load_c(n0 + BN);
       issue(ST ^ 1, n0 + BN);
     }
-    if (!CAUSAL || n0 <= qw + 31) {
+    if (!CAUSAL || n0 + (WK == 2 ? 32 * wt : 0) <= qw + 31) {
       tile_step(ST, n0, (n0 + BN > Lk) || (CAUSAL && n0 + BN - 1 > qw));
     }
   };
@@ -219,7 +229,11 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
     if (it + 1 < ntiles) iteration(it + 1, std::integral_constant<int, 1>{});
   }
 
-  if (!CAUSAL && p.rsplit > 1 &&
+  if constexpr (WK == 2) {
+    if (!pair_add<NDB, NG>([&](int i) SIGATTN_INLINE -> f32x16 & { return acc[i]; }, (float *)&sK[0][0], w, lane))
+      return;
+  }
+  if (WK == 1 && !CAUSAL && p.rsplit > 1 &&
       !split_combine<NDB, 4>([&](int i) SIGATTN_INLINE -> f32x16 & { return acc[i]; },
                              p.rs_part + (int64_t)ritem * p.rsplit * (BM * D), p.rs_cnt + ritem, rchunk,
                              p.rsplit, w, lane))
@@ -244,11 +258,12 @@ __device__ __forceinline__ void bwd_dq_body(const KParams &p, const int wg) {
   }
 }
 
-template <typename T, int D, bool CAUSAL, bool SCOREMOD>
+template <typename T, int D, int WK, bool CAUSAL, bool SCOREMOD>
 __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const KParams p) {
+  __shared__ __attribute__((aligned(16))) DqLds<D, SCOREMOD> lds;
   __shared__ unsigned long long gap_lds[2];
   const int wg = gap_prologue<2>(p, gap_lds);  // packed layouts: leading gap-zeroing workgroups
-  if (wg >= 0) bwd_dq_body<T, D, CAUSAL, SCOREMOD>(p, wg);
+  if (wg >= 0) bwd_dq_body<T, D, WK, CAUSAL, SCOREMOD>(p, wg, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -266,8 +281,11 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const KParams p) {
 // (causal diagonal, seq_lens_q, pipeline fill) are applied to the packed
 // words of the few blocks that need them.
 // ---------------------------------------------------------------------------
+template <int D> struct DkdvLds {
+  uint16_t q[4][64 * D], o[4][64 * D];
+};
 template <typename T, int D, bool CAUSAL, bool SCOREMOD, bool DSOUT>
-__device__ __forceinline__ void bwd_dkdv_body(const KParams &p, const int wg) {
+__device__ __forceinline__ void bwd_dkdv_body(const KParams &p, const int wg, DkdvLds<D> &lds) {
   constexpr int BN = 128;                 // keys per workgroup (32 per wave)
   constexpr int BMQ = 64;                 // queries per LDS tile (two 32-query blocks)
   constexpr int NST = 4;                  // LDS ring stages
@@ -282,8 +300,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const KParams &p, const int wg) {
   // indices need 4 tiles to be a whole number of ring turns.
   static_assert(4 % NST == 0, "ring stages");
 
-  __shared__ __attribute__((aligned(16))) uint16_t sQ[NST][BMQ * D];
-  __shared__ __attribute__((aligned(16))) uint16_t sO[NST][BMQ * D];
+  auto &sQ = lds.q;
+  auto &sO = lds.o;
 
   int b, h, kblk;
   int ritem = 0, rchunk = 0;  // range split: the item and this workgroup's chunk of its queries
@@ -618,19 +636,25 @@ __device__ __forceinline__ void bwd_dkdv_body(const KParams &p, const int wg) {
 
 template <typename T, int D, bool CAUSAL, bool SCOREMOD, bool DSOUT>
 __global__ __launch_bounds__(256, (D <= 64 ? 2 : 1)) void bwd_dkdv_kernel(const KParams p) {
-  bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, DSOUT>(p, blockIdx.x);
+  __shared__ __attribute__((aligned(16))) DkdvLds<D> lds;
+  bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, DSOUT>(p, blockIdx.x, lds);
 }
 
 // The recompute backward's two kernels in one launch (dense problems at
-// D <= 64 whose two grids together need at most one workgroup per CU): the
-// first ndq workgroups run dQ items, the rest dK/dV items, so the two halves
+// D <= 64 whose two grids of 128-row blocks together need at most one workgroup
+// per CU): the first ndq workgroups run dQ items, in pairs of waves as
+// launch_bwd_dq_mfma runs these grids, the rest dK/dV items, so the two halves
 // share the GPU instead of each leaving half of it idle.  The bodies are the
-// kernels' own, so results are bit-identical to the two launches.  The two
-// bodies' LDS adds up (96 KB at D = 64), so one workgroup fits per CU.
+// kernels' own, so results are bit-identical to the two launches.  They share
+// their LDS, and two workgroups fit a CU.
 template <typename T, int D, bool CAUSAL, bool SCOREMOD>
-__global__ __launch_bounds__(256, 1) void bwd_fused_kernel(const KParams pq, const KParams pk, int ndq) {
-  if ((int)blockIdx.x < ndq) bwd_dq_body<T, D, CAUSAL, SCOREMOD>(pq, blockIdx.x);
-  else bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, false>(pk, (int)blockIdx.x - ndq);
+__global__ __launch_bounds__(256, 2) void bwd_fused_kernel(const KParams pq, const KParams pk, int ndq) {
+  __shared__ __attribute__((aligned(16))) union {
+    DqLds<D, SCOREMOD> dq;
+    DkdvLds<D> dkdv;
+  } lds;
+  if ((int)blockIdx.x < ndq) bwd_dq_body<T, D, 2, CAUSAL, SCOREMOD>(pq, blockIdx.x, lds.dq);
+  else bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, false>(pk, (int)blockIdx.x - ndq, lds.dkdv);
 }
 
 // ---------------------------------------------------------------------------
@@ -1290,20 +1314,35 @@ static void launch_rows(const KParams &kp, int rows, Launch &&launch) {
   launch(p, dim3((unsigned)(p.nblk * p.B * p.H)));
 }
 
-template <typename T, int D>
-static void bwd_dq_t(const KParams &kp, bool causal, bool sm, hipStream_t st) {
-  launch_rows<128>(kp, kp.Tq, [&](const KParams &p, dim3 grid) {
+template <typename T, int D, int WK>
+static void bwd_dq_w(const KParams &kp, bool causal, bool sm, hipStream_t st) {
+  launch_rows<128 / WK>(kp, kp.Tq, [&](const KParams &p, dim3 grid) {
     // Range split (dense non-causal): rsplit workgroups per item.
-    if (!causal && p.rsplit > 1) grid.x *= (unsigned)p.rsplit;
+    if (WK == 1 && !causal && p.rsplit > 1) grid.x *= (unsigned)p.rsplit;
     grid.x += (unsigned)(p.ngap[0] + p.ngap[1]);
     if (causal) {
-      if (sm) bwd_dq_kernel<T, D, true, true><<<grid, 256, 0, st>>>(p);
-      else bwd_dq_kernel<T, D, true, false><<<grid, 256, 0, st>>>(p);
+      if (sm) bwd_dq_kernel<T, D, WK, true, true><<<grid, 256, 0, st>>>(p);
+      else bwd_dq_kernel<T, D, WK, true, false><<<grid, 256, 0, st>>>(p);
     } else {
-      if (sm) bwd_dq_kernel<T, D, false, true><<<grid, 256, 0, st>>>(p);
-      else bwd_dq_kernel<T, D, false, false><<<grid, 256, 0, st>>>(p);
+      if (sm) bwd_dq_kernel<T, D, WK, false, true><<<grid, 256, 0, st>>>(p);
+      else bwd_dq_kernel<T, D, WK, false, false><<<grid, 256, 0, st>>>(p);
     }
   });
+}
+
+// Pairs of waves (WK = 2, D <= 64) halve the longest item's chain for twice the
+// tile copies.  Causal and ragged grids end with their longest items, so they
+// gain up to four 128-row blocks per CU (fp16 causal B=8 Lmax=2048 H=8 D=64,
+// lengths 641..2048, 1024 blocks: 50.7 -> 41.5 us); equal items gain only where
+// they leave CUs idle (B=4 T=1500 H=16 D=64 non-causal, 768 blocks, forward +
+// backward: 211 -> 216 us).
+template <typename T, int D>
+static void bwd_dq_t(const KParams &kp, bool causal, bool sm, hipStream_t st) {
+  if constexpr (D <= 64) {
+    if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, causal || kp.ragged() ? 4 : 1))
+      return bwd_dq_w<T, D, 2>(kp, causal, sm, st);
+  }
+  bwd_dq_w<T, D, 1>(kp, causal, sm, st);
 }
 
 template <typename T, int D, bool DSOUT>
@@ -1431,7 +1470,7 @@ void launch_bwd_fused_mfma(const KParams &kp, int dtype, int D, bool causal, boo
     constexpr int DD = decltype(d)::value;
     if constexpr (DD <= 64) {
       KParams pq = kp, pk = kp;
-      pq.nblk = (kp.Tq + 127) / 128;
+      pq.nblk = (kp.Tq + 63) / 64;
       pk.nblk = (kp.Tk + 127) / 128;
       pq.rsplit = pk.rsplit = 1;
       pq.ngap[0] = pq.ngap[1] = pk.ngap[0] = pk.ngap[1] = 0;  // dense problems only: no packed gap rows

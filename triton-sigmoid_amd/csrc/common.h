@@ -866,7 +866,46 @@ template <int D> struct TileOffsets {
       tr_op[db][1] = toff<D>(row + 8, col);
     }
   }
+  // Moves every offset down by `rows` rows, a multiple of 16.
+  __device__ __forceinline__ void advance(int rows) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) row_op[ks] += rows * D;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) tr_op[db][0] += rows * D, tr_op[db][1] += rows * D;
+  }
 };
+
+// Adds the accumulators (NACC f32x16 per lane, acc(i)) of the workgroup's
+// waves NG .. 2·NG-1 into waves 0 .. NG-1, which hold the same rows, through
+// LDS that holds NG · NACC · 4 KB and that no wave reads or fills any more once
+// all have arrived here.  All 2·NG waves call it; false for the second half,
+// which has nothing left to do.
+template <int NACC, int NG, class Acc>
+__device__ __forceinline__ bool pair_add(Acc &&acc, float *lds, int w, int lane) {
+  float *at = lds + (w % NG) * NACC * 1024 + 4 * lane;
+  __syncthreads();
+  if (w >= NG) {
+#pragma unroll
+    for (int i = 0; i < NACC; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16 &a = acc(i);
+        *(f32x4 *)(at + (4 * i + g) * 256) = (f32x4){a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+      }
+    __syncthreads();
+    return false;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NACC; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x16 &a = acc(i);
+      const f32x4 v = *(const f32x4 *)(at + (4 * i + g) * 256);
+      a[4 * g] += v.x, a[4 * g + 1] += v.y, a[4 * g + 2] += v.z, a[4 * g + 3] += v.w;
+    }
+  return true;
+}
 
 // Operand read at row (row16 + l%32) where row16 is a multiple of 16.
 template <int D>

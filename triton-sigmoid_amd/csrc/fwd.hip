@@ -38,7 +38,7 @@ namespace sigattn {
 #define SIGATTN_FWD_D64_STAGES 3
 #endif
 
-template <int D> constexpr int fwd_stages() { return D == 64 ? SIGATTN_FWD_D64_STAGES : 4; }
+template <int D, int WK = 1> constexpr int fwd_stages() { return D == 64 && WK == 1 ? SIGATTN_FWD_D64_STAGES : 4; }
 
 // Dense causal grids pair query blocks (j, nblk-1-j) in one workgroup, in
 // the XCD-grouped order (every workgroup equal; K / V of a (batch, head) read
@@ -62,18 +62,22 @@ constexpr bool kFwdCausalPairs = SIGATTN_FWD_CAUSAL_PAIRS != 0;
 constexpr int kFwdBhGroup = SIGATTN_FWD_BH_GROUP;
 // Resident workgroups per CU: D = 128 one (128 KB of LDS); D = 64 three (or
 // two with four stages); D = 32 four (32 KB, at most 128 registers per wave).
-template <int D> constexpr int fwd_occupancy() {
-  return D == 64 ? (fwd_stages<D>() == 3 ? 3 : 2) : (D == 32 ? 4 : 1);
+template <int D, int WK = 1> constexpr int fwd_occupancy() {
+  return D == 64 ? (fwd_stages<D, WK>() == 3 ? 3 : 2) : (D == 32 ? 4 : 1);
 }
 
-template <typename T, int D, int NWV, int NCB, bool CAUSAL, bool SCOREMOD>
-__global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(const KParams p) {
+template <typename T, int D, int NWV, int NCB, int WK, bool CAUSAL, bool SCOREMOD>
+__global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK>())) void fwd_mfma_kernel(const KParams p) {
   // NWV waves per workgroup (8: two per SIMD), NCB 32-query column blocks each.
+  // WK = 2: the waves form pairs that hold the same queries; wave `wt` of a
+  // pair takes block wt of every 64-key tile (one region per tile instead of
+  // two) and the pair's accumulators are added at the end.
   constexpr int QW = 32 * NCB;          // queries per wave
-  constexpr int BM = NWV * QW;          // queries per workgroup
+  constexpr int NG = NWV / WK;          // query groups
+  constexpr int BM = NG * QW;           // queries per workgroup
   constexpr int BN = 64;                // keys per LDS tile (two 32-key blocks)
   // LDS ring stages: D = 64 uses three (48 KB), so three workgroups share a CU.
-  constexpr int NST = fwd_stages<D>();
+  constexpr int NST = fwd_stages<D, WK>();
   constexpr int NKS = D / 16;           // MFMA k-steps over the head dim
   constexpr int NDB = D / 32;           // 32-row blocks of Oᵀ
   constexpr int NSTEP = NKS + 2 * NDB;  // steps (NCB MFMAs sharing an A operand) per region
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
   if (wg < 0) return;
   int b, h, qb0, nitems = 1;
   int ritem = 0, rchunk = 0;  // range split: the item and this workgroup's chunk of its keys
-  if (!CAUSAL && p.rsplit > 1) {
+  if (WK == 1 && !CAUSAL && p.rsplit > 1) {
     // Small dense grids: the rsplit workgroups of an item take adjacent ids.
     int bh;
     ritem = wg / p.rsplit, rchunk = wg % p.rsplit;
@@ -105,7 +109,7 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     const auto lq = [&](int i) SIGATTN_INLINE { return p.len_q(i); };
     const auto lk = [&](int i) SIGATTN_INLINE { return p.len_k(i); };
     const WorkItem it = CAUSAL ? WorkOrder::by_level(wg, p.B, p.H, lq, BM, p.nblk, true, p.ncu,
-                                                     fwd_occupancy<D>())
+                                                     fwd_occupancy<D, WK>())
                                : WorkOrder::by_stream(wg, p.B, p.H, lq, BM, p.nblk, lk);
     b = it.b, h = it.h, qb0 = it.blk;
   } else {
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     // Keys of this workgroup: under the range split, its chunk of the item's
     // key tiles, indexed from the chunk's first key.
     int key0 = 0, Lk = p.len_k(b);
-    if (!CAUSAL && p.rsplit > 1) {
+    if (WK == 1 && !CAUSAL && p.rsplit > 1) {
       const int ntk = (Lk + BN - 1) / BN;
       key0 = split_tile(rchunk, p.rsplit, ntk) * BN;
       Lk = min(Lk, split_tile(rchunk + 1, p.rsplit, ntk) * BN) - key0;
@@ -165,7 +169,8 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     // Query slot of the wave.  With eight waves, waves w and w+4 share a SIMD;
     // giving them complementary slots (w and 7-w) evens out the per-SIMD work of
     // causal diagonal workgroups once waves stop at their own last key block.
-    const int slot = (NWV == 8 && w >= 4) ? 11 - w : w;
+    const int wt = w / NG;  // place in the wave's pair (WK = 2)
+    const int slot = WK == 2 ? w % NG : ((NWV == 8 && w >= 4) ? 11 - w : w);
     const int qw = q0 + slot * QW;    // this wave's first query
     const int myq0 = qw + l32;        // this lane's query in column block 0 (block c: +32c)
 
@@ -212,6 +217,7 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
 
     TileOffsets<D> to;
     to.init(lane);
+    if constexpr (WK == 2) to.advance(32 * wt);  // this wave's half of every tile
     DmaPlan<BN, D, NWV> dma;
     dma.init(w, lane, half);
     const int kv_stride_bytes = (int)(p.sk_t * 2);
@@ -267,6 +273,9 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     u32x4 opq[LA];              // A operands of the next LA steps (slot = step % LA)
     float ea[2];                // exp2 terms of the next word (sigmoid stage A)
 
+    // 32-key block that the wave's region r computes S of.
+    auto block_of = [&](int r) SIGATTN_INLINE { return WK == 2 ? 2 * r + wt : r; };
+
     // Region r (U = r mod 8, so every slot and ring stage is static):
     //   MFMA: Sᵀ(r) = K·Qᵀ and Oᵀ += Vᵀ·Pᵀ(r-2), one step = NCB MFMAs (one per
     //         column block) sharing an A operand read LA steps earlier;
@@ -283,11 +292,13 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     auto region = [&](int r, auto u_tag) SIGATTN_INLINE {
       constexpr int U = decltype(u_tag)::value;
       constexpr int SL = U % 2;                    // parity of blocks r and r-2
-      constexpr int KL = 32 * (U % 2), KLn = 32 * ((U + 1) % 2);
-      constexpr int STC = (U / 2) % NST;           // stage of block r
-      constexpr int STV = ((U + 2 * NST - 2) / 2) % NST;  // stage of block r-2
-      constexpr int STCn = ((U + 1) / 2) % NST;    // stage of block r+1
-      constexpr int STVn = ((U + 2 * NST - 1) / 2) % NST;  // stage of block r-1
+      constexpr int RPT = 2 / WK;                  // regions per tile
+      constexpr int KL = WK == 2 ? 0 : 32 * (U % 2), KLn = WK == 2 ? 0 : 32 * ((U + 1) % 2);
+      constexpr int STC = (U / RPT) % NST;         // stage of block r
+      constexpr int STV = ((U + 2 * NST - 2) / RPT) % NST;  // stage of block r-2
+      constexpr int STCn = ((U + 1) / RPT) % NST;  // stage of block r+1
+      constexpr int STVn = ((U + 2 * NST - 1) / RPT) % NST;  // stage of block r-1
+      const int cl = WK == 2 ? 32 * wt : 0;        // this wave's half of sC's tiles
       f32x16(&sc)[NCB] = sbuf[SL];
       const f32x16(&sp)[NCB] = sbuf[1 - SL];
       uint32_t(&pn)[NCB][8] = pbuf[1 - SL];
@@ -297,11 +308,11 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
       if constexpr (SCOREMOD) {
   #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const float4 cv = *(const float4 *)&sC[STVn * BN + KLn + 8 * g + 4 * hi];
+          const float4 cv = *(const float4 *)&sC[STVn * BN + KLn + cl + 8 * g + 4 * hi];
           c[4 * g + 0] = cv.x; c[4 * g + 1] = cv.y; c[4 * g + 2] = cv.z; c[4 * g + 3] = cv.w;
         }
   #pragma unroll
-        for (int i = 0; i < 2; ++i) cn[i] = sC[STC * BN + KL + 4 * hi + i];
+        for (int i = 0; i < 2; ++i) cn[i] = sC[STC * BN + KL + cl + 4 * hi + i];
       } else {
   #pragma unroll
         for (int i = 0; i < 16; ++i) c[i] = nbl;
@@ -309,14 +320,15 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
       }
   #pragma unroll
       for (int step = 0; step < NSTEP; ++step) {
-        if ((U % 2) == 1 && step == BAR) {
-          const int u = (r + 1) / 2;
+        if ((WK == 2 || (U % 2) == 1) && step == BAR) {
+          const int u = (r + 1) / RPT;
           if (u < ntiles) {
             wait_dma();
             if (SCOREMOD && tid < BN) sC[(u % NST) * BN + tid] = creg;
-            // With three stages the copy below refills the stage this region's
-            // Vᵀ operands came from: every wave's reads of it complete first.
-            if constexpr (NST == 3) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            // With three stages (four when a region is a tile) the copy below
+            // refills the stage this region's Vᵀ operands came from: every
+            // wave's reads of it complete first.
+            if constexpr (NST == 3 || WK == 2) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -368,7 +380,7 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (r == 0 || needs_mask(r - 1)) mask_words(pn, r - 1);
+      if (r == 0 || needs_mask(block_of(r - 1))) mask_words(pn, block_of(r - 1));
     };
 
     // Pipeline fill: Pᵀ(-2) = Pᵀ(-1) = 0 (the latter through its mask).  The
@@ -385,7 +397,11 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
       }
     }
     ea[0] = ea[1] = 0.0f;
-    for (int i = tid; i < BN * D / 8; i += 64 * NWV) *(u32x4 *)&sV[NST - 1][8 * i] = zero4();
+    for (int i = tid; i < BN * D / 8; i += 64 * NWV) {
+      *(u32x4 *)&sV[NST - 1][8 * i] = zero4();
+      // A region per tile: blocks -2 and -1 are tiles -2 and -1.
+      if constexpr (WK == 2) *(u32x4 *)&sV[NST - 2][8 * i] = zero4();
+    }
 
     if (ntiles > 0) {
       issue(0, 0);
@@ -400,25 +416,29 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
     // This wave computes only up to its own last visible key block (causal) and
     // not at all past seq_lens_q; afterwards it only takes part in the tile
     // barriers and copies, leaving its SIMD to the other wave there.
-    int NBw = NB;
-    if (CAUSAL) NBw = min(NBw, (qw + QW - 1) / 32 + 1);
+    int NBw = WK == 2 ? ntiles : NB;
+    if (CAUSAL) {
+      const int last = (qw + QW - 1) / 32;  // the wave's last visible block
+      NBw = min(NBw, WK == 2 ? (last >= wt ? (last - wt) / 2 + 1 : 0) : last + 1);
+    }
     if (qw >= Lq) NBw = 0;
     const int RW = NBw > 0 ? NBw + 2 : 0;
-    // One pass of the loop covers 2·NST regions (NST tiles), so region r0 + U
-    // starts tile r0/2 + U/2 with r0/2 a multiple of NST: every stage index in
-    // region() is a compile-time function of U.
-    for (int r0 = 0; r0 < RW; r0 += 2 * NST) {
-      Unroll<0, 2 * NST>::run([&](auto u) SIGATTN_INLINE {
+    // One pass of the loop covers NST tiles (2·NST regions, NST with a region
+    // per tile), so every stage index in region() is a compile-time function
+    // of U.
+    constexpr int UN = 2 * NST / WK;
+    for (int r0 = 0; r0 < RW; r0 += UN) {
+      Unroll<0, UN>::run([&](auto u) SIGATTN_INLINE {
         if (r0 + decltype(u)::value < RW) region(r0 + decltype(u)::value, u);
       });
     }
     // The rest of the workgroup's regions: the same barriers and copies.
-    for (int r = RW | 1; r < NB + 2; r += 2) {
-      const int u = (r + 1) / 2;
+    for (int r = WK == 2 ? RW : (RW | 1); r < NB / WK + 2; r += 2 / WK) {
+      const int u = (r + 1) * WK / 2;
       if (u < ntiles) {
         wait_dma();
         if (SCOREMOD && tid < BN) sC[(u % NST) * BN + tid] = creg;
-        if constexpr (NST == 3) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if constexpr (NST == 3 || WK == 2) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -426,7 +446,15 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
       }
     }
 
-    if (!CAUSAL && p.rsplit > 1 &&
+    if constexpr (WK == 2) {
+      // The pair's second wave hands its accumulators to the first.
+      static_assert(!(CAUSAL && kFwdCausalPairs), "one query block per workgroup");
+      if (!pair_add<NCB * NDB, NG>([&](int i) SIGATTN_INLINE -> f32x16 & { return acc[i / NDB][i % NDB]; },
+                                   (float *)&sK[0][0], w, lane))
+        return;
+    }
+
+    if (WK == 1 && !CAUSAL && p.rsplit > 1 &&
         !split_combine<NCB * NDB, NWV>([&](int i) SIGATTN_INLINE -> f32x16 & { return acc[i / NDB][i % NDB]; },
                                        p.rs_part + (int64_t)ritem * p.rsplit * (BM * D), p.rs_cnt + ritem,
                                        rchunk, p.rsplit, w, lane))
@@ -465,9 +493,9 @@ __global__ __launch_bounds__(64 * NWV, fwd_occupancy<D>()) void fwd_mfma_kernel(
 #define SIGATTN_FWD_NCB 1
 #endif
 
-template <typename T, int D, int NWV>
+template <typename T, int D, int NWV, int WK>
 static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  constexpr int NCB = SIGATTN_FWD_NCB, BM = NWV * 32 * NCB;
+  constexpr int NCB = SIGATTN_FWD_NCB, BM = NWV * 32 * NCB / WK;
   KParams p = kp;
   p.nblk = (p.Tq + BM - 1) / BM;
   // Dense causal problems (the kernel's order when not ragged with B <= 64):
@@ -477,11 +505,11 @@ static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStrea
   const dim3 grid((unsigned)((pairs ? (p.nblk + 1) / 2 : p.nblk) * p.B * p.H * p.rsplit + p.ngap[0] + p.ngap[1]));
   const dim3 block(64 * NWV);
   if (causal) {
-    if (scoremod) fwd_mfma_kernel<T, D, NWV, NCB, true, true><<<grid, block, 0, st>>>(p);
-    else fwd_mfma_kernel<T, D, NWV, NCB, true, false><<<grid, block, 0, st>>>(p);
+    if (scoremod) fwd_mfma_kernel<T, D, NWV, NCB, WK, true, true><<<grid, block, 0, st>>>(p);
+    else fwd_mfma_kernel<T, D, NWV, NCB, WK, true, false><<<grid, block, 0, st>>>(p);
   } else {
-    if (scoremod) fwd_mfma_kernel<T, D, NWV, NCB, false, true><<<grid, block, 0, st>>>(p);
-    else fwd_mfma_kernel<T, D, NWV, NCB, false, false><<<grid, block, 0, st>>>(p);
+    if (scoremod) fwd_mfma_kernel<T, D, NWV, NCB, WK, false, true><<<grid, block, 0, st>>>(p);
+    else fwd_mfma_kernel<T, D, NWV, NCB, WK, false, false><<<grid, block, 0, st>>>(p);
   }
 }
 
@@ -493,7 +521,15 @@ static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStrea
 // and 5-13 % padded.
 template <typename T, int D>
 static void launch_fwd_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  launch_fwd_w<T, D, (D <= 64 ? 4 : 8) / SIGATTN_FWD_NCB>(kp, causal, scoremod, st);
+  // Pairs of waves (WK = 2) where the 128-query blocks number at most one per
+  // CU: half of every block's chain (fp16 B=2 T=1024 H=8 D=64, 128 blocks: call
+  // 16.8 -> 12.2 us).  Beyond, a tile per region leaves its copy one region of
+  // time and the fourth stage the third workgroup (512 blocks 27.6 -> 31.2 us
+  // non-causal, 19.8 -> 22.3 causal).
+  if constexpr (D <= 64) {
+    if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, 1)) return launch_fwd_w<T, D, 4, 2>(kp, causal, scoremod, st);
+  }
+  launch_fwd_w<T, D, (D <= 64 ? 4 : 8) / SIGATTN_FWD_NCB, 1>(kp, causal, scoremod, st);
 }
 
 int fwd_rows_per_workgroup(int D) { return (D <= 64 ? 4 : 8) * 32; }

@@ -19,6 +19,13 @@ int device_compute_units();
 // Rows per workgroup and resident workgroups per CU of the MFMA forward and
 // of the recompute backward's kernels (D in {64, 128}); the range split of
 // small dense grids (KParams::rsplit) sizes itself from them.
+// At most `per_cu` 128-row blocks per compute unit: where the D <= 64 forward
+// and dQ kernels let two waves share each 32 rows (half the chain per workgroup,
+// twice the workgroups).
+inline bool wave_pairs(const KParams &p, int rows, int per_cu) {
+  return (int64_t)p.B * p.H * ((rows + 127) / 128) <= per_cu * (int64_t)p.ncu;
+}
+
 int fwd_rows_per_workgroup(int D);
 int fwd_workgroups_per_cu(int D);
 int bwd_dq_rows_per_workgroup();

@@ -176,7 +176,9 @@ def sigmoid_attention_varlen(
 
     Returns:
         [total_q, H, D] output, equal row for row to what
-        `sigmoid_attention_padded` returns for the same sequences.
+        `sigmoid_attention_padded` returns for the same sequences (within
+        fp32 summation order where the longest sequence and the padded length
+        fall on two sides of a kernel's size rule).
 
     Rows outside every sequence -- before cu[0], past cu[B] when cu does not
     cover all rows, and past max_seqlen of a longer sequence -- are zeros in
