@@ -423,3 +423,27 @@ def test_default_bias_kernel_equals_the_operators(B):
                    (_capi.default_bias(dev, cu_seqlens=cu), cu[1:] - cu[:-1])):
         want = -torch.log(n.to(torch.float32))
         assert got.shape == (B,) and torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("B,H,T", [(3, 5, 257), (8, 16, 300), (16, 16, 385)])  # 90, 768 and 2048 blocks of 128 rows
+@pytest.mark.parametrize("padded", [False, True])
+def test_one_launch_causal_backward_equals_the_two_kernels(D, B, H, T, padded):
+    """Causal dense and padded grids run dK/dV and dQ in one launch up to six
+    128-row blocks per compute unit: the same bits as the kernels apart."""
+    g = torch.Generator().manual_seed(T + D)
+    q, k, v, do = (randn((B, T, H, D), torch.bfloat16, DEV, g) for _ in range(4))
+    lens = torch.randint(0, T + 1, (B,), generator=g, dtype=torch.int32).to(DEV) if padded else None
+    bias = torch.full((B,), -2.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    lib = _capi.load_library()
+    pr = _capi._problem(q, k, v, bias, None, scale, lens, lens, True)
+    one = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    two = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.sigattn_bwd(ctypes.byref(pr), do.data_ptr(), *(t.data_ptr() for t in one), stream) == 0
+    assert lib.sigattn_bwd_dq(ctypes.byref(pr), do.data_ptr(), two[0].data_ptr(), stream) == 0
+    assert lib.sigattn_bwd_dkdv(ctypes.byref(pr), do.data_ptr(), two[1].data_ptr(), two[2].data_ptr(), stream) == 0
+    torch.cuda.synchronize()
+    for a, b in zip(one, two):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

@@ -640,21 +640,21 @@ __global__ __launch_bounds__(256, (D <= 64 ? 2 : 1)) void bwd_dkdv_kernel(const 
   bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, DSOUT>(p, blockIdx.x, lds);
 }
 
-// The recompute backward's two kernels in one launch (dense problems at
-// D <= 64 whose two grids of 128-row blocks together need at most one workgroup
-// per CU): the first ndq workgroups run dQ items, in pairs of waves as
-// launch_bwd_dq_mfma runs these grids, the rest dK/dV items, so the two halves
-// share the GPU instead of each leaving half of it idle.  The bodies are the
-// kernels' own, so results are bit-identical to the two launches.  They share
-// their LDS, and two workgroups fit a CU.
+// The recompute backward's two kernels in one launch: the first nkv workgroups
+// run dK/dV items, the rest dQ items, in pairs of waves as launch_bwd_dq_mfma
+// runs these grids.  On grids within one workgroup per CU the two halves share
+// the GPU instead of each leaving half of it idle; on causal ones of several,
+// the short dQ items run beside the dK/dV kernel's last ones.  The bodies are
+// the kernels' own, so results are bit-identical to the two launches.  They
+// share their LDS, and two workgroups fit a CU.
 template <typename T, int D, bool CAUSAL, bool SCOREMOD>
-__global__ __launch_bounds__(256, 2) void bwd_fused_kernel(const KParams pq, const KParams pk, int ndq) {
+__global__ __launch_bounds__(256, 2) void bwd_fused_kernel(const KParams pq, const KParams pk, int nkv) {
   __shared__ __attribute__((aligned(16))) union {
     DqLds<D, SCOREMOD> dq;
     DkdvLds<D> dkdv;
   } lds;
-  if ((int)blockIdx.x < ndq) bwd_dq_body<T, D, 2, CAUSAL, SCOREMOD>(pq, blockIdx.x, lds.dq);
-  else bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, false>(pk, (int)blockIdx.x - ndq, lds.dkdv);
+  if ((int)blockIdx.x < nkv) bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, false>(pk, blockIdx.x, lds.dkdv);
+  else bwd_dq_body<T, D, 2, CAUSAL, SCOREMOD>(pq, (int)blockIdx.x - nkv, lds.dq);
 }
 
 // ---------------------------------------------------------------------------
@@ -1473,15 +1473,15 @@ void launch_bwd_fused_mfma(const KParams &kp, int dtype, int D, bool causal, boo
       pq.nblk = (kp.Tq + 63) / 64;
       pk.nblk = (kp.Tk + 127) / 128;
       pq.rsplit = pk.rsplit = 1;
-      pq.ngap[0] = pq.ngap[1] = pk.ngap[0] = pk.ngap[1] = 0;  // dense problems only: no packed gap rows
-      const int ndq = pq.nblk * kp.B * kp.H;
-      const dim3 grid((unsigned)(ndq + pk.nblk * kp.B * kp.H));
+      pq.ngap[0] = pq.ngap[1] = pk.ngap[0] = pk.ngap[1] = 0;  // no packed layouts: no gap rows
+      const int nkv = pk.nblk * kp.B * kp.H;
+      const dim3 grid((unsigned)(nkv + pq.nblk * kp.B * kp.H));
       if (causal) {
-        if (sm) bwd_fused_kernel<T, DD, true, true><<<grid, 256, 0, st>>>(pq, pk, ndq);
-        else bwd_fused_kernel<T, DD, true, false><<<grid, 256, 0, st>>>(pq, pk, ndq);
+        if (sm) bwd_fused_kernel<T, DD, true, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
+        else bwd_fused_kernel<T, DD, true, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
       } else {
-        if (sm) bwd_fused_kernel<T, DD, false, true><<<grid, 256, 0, st>>>(pq, pk, ndq);
-        else bwd_fused_kernel<T, DD, false, false><<<grid, 256, 0, st>>>(pq, pk, ndq);
+        if (sm) bwd_fused_kernel<T, DD, false, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
+        else bwd_fused_kernel<T, DD, false, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
       }
     }
   });

@@ -165,15 +165,25 @@ bool is_ragged(const sigattn_problem *p) {
 }
 
 // The recompute backward's dQ and dK/dV kernels run as one launch
-// (launch_bwd_fused_mfma) when the problem is dense, its 16-bit kernel
-// instance has D <= 64, and the two grids (128 rows per workgroup) together
-// need at most one workgroup per CU: apart, each would leave the CUs the
-// other needs idle.
+// (launch_bwd_fused_mfma) where the 16-bit kernel instance has D <= 64 and
+//   * the problem is dense and the two grids (128 rows per workgroup)
+//     together need at most one workgroup per CU: apart, each would leave the
+//     CUs the other needs idle; or
+//   * it is causal and not packed, with at most six such workgroups per CU
+//     (and no more dQ ones than launch_bwd_dq_mfma runs in pairs of waves, the
+//     one-launch kernel's form): each kernel alone ends with few CUs busy.
+//     Forward + backward, us, apart / one launch: B=1 T=8000 H=8 D=64, four
+//     per CU, 398 / 371; B=2 T=2048 H=16 D=32, four, 99.4 / 89.7; B=4 T=1500
+//     H=16 D=64, six, 138.6 / 133.8; B=8 T=2048 H=8 D=64, eight, 223 / 234 (dQ
+//     then misses its third workgroup per CU).
+constexpr int64_t kFuseCausal = 6;
 bool fuse_backward(const sigattn_problem *p) {
-  if (is_ragged(p) || mfma_head_dim(p) > 64) return false;
+  if (p->cu_seqlens_q != nullptr || p->cu_seqlens_k != nullptr || mfma_head_dim(p) > 64) return false;
   const int64_t cus = sigattn::device_compute_units();
-  const int64_t wgs = p->B * p->H * (cdiv(p->Tq, 128) + cdiv(p->Tk, 128));
-  return cus > 0 && wgs <= cus;
+  const int64_t ndq = p->B * p->H * cdiv(p->Tq, 128), nkv = p->B * p->H * cdiv(p->Tk, 128);
+  if (cus <= 0) return false;
+  if (!is_ragged(p) && ndq + nkv <= cus) return true;
+  return p->causal != 0 && ndq > 0 && nkv > 0 && ndq + nkv <= kFuseCausal * cus && ndq <= 4 * cus;
 }
 
 // The recompute backward's dQ and dK/dV kernels run concurrently, dK/dV on a
