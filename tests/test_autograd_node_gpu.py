@@ -222,3 +222,57 @@ def test_saved_tensor_hooks_give_plain_gradients(case, hook, binding, monkeypatc
     del junk
     for name, x, y in zip(("O", "dQ", "dK", "dV"), [o.detach()] + [t.grad for t in leaves], want):
         assert torch.equal(x, y), f"{name} under {hook} ({binding} node) differs from the plain backward"
+
+
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("kind", ["default", "scale", "bias", "mod", "int-lens", "strided", "no-lens", "float-mod"])
+def test_quick_entry_equals_the_python_layer(monkeypatch, padded, kind):
+    """The node's entry for canonical calls against the Python layer: the same
+    bits in O and the gradients, and None (the layer takes over) for the rest."""
+    B, T, H, D = 3, 130, 2, 64
+    g = torch.Generator().manual_seed(4)
+    q, k, v, do = (randn((B, T, H, D), torch.bfloat16, DEV, g) for _ in range(4))
+    lens = torch.tensor([130, 1, 77], dtype=torch.int64 if kind == "int-lens" else torch.int32, device=DEV)
+    kw = {"scale": dict(scale=0.2), "bias": dict(sigmoid_bias=-1.5),
+          "mod": dict(score_mod=torch.randn((B, T), generator=g).to(DEV)),
+          "float-mod": dict(score_mod=torch.randn((B, T), generator=g).to(DEV, torch.float16))}.get(kind, {})
+    if kind == "strided":
+        q = q.transpose(1, 2).contiguous().transpose(1, 2)
+
+    def run():
+        ins = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        if padded:
+            ln = {} if kind == "no-lens" else dict(seq_lens_k=lens, seq_lens_q=lens)
+            o = ts.sigmoid_attention_padded(*ins, is_causal=True, **ln, **kw)
+        else:
+            o = ts.sigmoid_attention(*ins, is_causal=True, **kw)
+        return (o, *torch.autograd.grad(o, ins, do))
+
+    assert _capi.autograd_node() is not None and _capi.quick is not None
+    took = []
+    real = _capi.quick
+    monkeypatch.setattr(_capi, "quick", lambda *a: took.append(real(*a)) or took[-1])
+    got = run()
+    monkeypatch.setattr(_capi, "quick", None)
+    want = run()
+    assert len(took) == 1
+    refused = kind in ("strided", "float-mod") or (padded and kind == "int-lens")
+    assert (took[0] is None) == refused
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_quick_entry_leaves_errors_and_overrides_to_the_python_layer(monkeypatch):
+    q = torch.randn((1, 8, 2, 32), device=DEV, dtype=torch.float16)
+    ts.sigmoid_attention(q, q, q)
+    assert _capi.quick(q, q, q, None, None, False, False, None, None, None) is not None
+    for bad in (q[0], q[:, :, :, :16], q.double(), q.cpu(), q[:, :0], None, 3):
+        assert _capi.quick(bad, q, q, None, None, False, False, None, None, None) is None
+    assert _capi.quick(q, q, q, None, None, False, 1, None, None, None) is None
+    assert _capi.quick(q, q, q, None, None, False, False, torch.tensor(1.0), None, None) is None
+    with pytest.raises(ValueError, match="4D"):
+        ts.sigmoid_attention(q[0], q, q)
+    for name, value in (("SIGATTN_EAGER_BINDING", "python"), ("SIGATTN_BWD_WORKSPACE_MB", "0")):
+        monkeypatch.setenv(name, value)
+        assert _capi.quick(q, q, q, None, None, False, False, None, None, None) is None
+        monkeypatch.delenv(name)

@@ -31,8 +31,13 @@
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
+#include <cmath>
+#include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/sigattn.h"
@@ -45,6 +50,7 @@ using torch::autograd::tensor_list;
 
 struct Api {
   decltype(&sigattn_strerror) strerror = nullptr;
+  decltype(&sigattn_default_bias) default_bias = nullptr;
   decltype(&sigattn_fwd_workspace_bytes) fwd_workspace_bytes = nullptr;
   decltype(&sigattn_fwd_ws) fwd_ws = nullptr;
   decltype(&sigattn_fwd_decode_workspace_bytes) fwd_decode_workspace_bytes = nullptr;
@@ -256,6 +262,113 @@ Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor
                             cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k);
 }
 
+// The eager public APIs' calls with canonical arguments, without the Python
+// layer's per-call checks and conversions (about 6 of 12 us of host time, which
+// is what a small call takes): exact torch.Tensors, contiguous, one gfx950
+// device, matching shapes, plain numbers, no environment overrides, no stream
+// capture.  Everything else -- and so every error -- is None, and the Python
+// layer takes the call.
+struct Quick {
+  // Constants [n] on a device, as _capi.device_constant keeps them: made by a
+  // blocking copy, at most kMax, never freed (a queued kernel may read one).
+  static constexpr size_t kMax = 256;
+  static Tensor constant(int64_t n, double value, at::ScalarType type, const at::Device &dev) {
+    static std::mutex mu;
+    static auto *kept = new std::map<std::tuple<int, int64_t, double, int>, Tensor>;  // outlives every thread
+    const std::tuple<int, int64_t, double, int> key(dev.index(), n, value, (int)type);
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = kept->find(key);
+    if (it != kept->end()) return it->second;
+    if (kept->size() >= kMax || std::isnan(value)) return Tensor();
+    const auto opt = at::TensorOptions().dtype(type);
+    const Tensor t = (n < 0 ? at::full({}, value, opt) : at::full({n}, value, opt)).to(dev);
+    kept->emplace(key, t);
+    return t;
+  }
+  static bool gfx950(int dev) {
+    static std::atomic<int> known[64];  // 0: not looked at, 1: gfx950, 2: another
+    if (dev < 0 || dev >= 64) return false;
+    int v = known[dev].load(std::memory_order_relaxed);
+    if (v == 0) {
+      hipDeviceProp_t prop;
+      if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return false;
+      v = std::strncmp(prop.gcnArchName, "gfx950", 6) == 0 ? 1 : 2;
+      known[dev].store(v, std::memory_order_relaxed);
+    }
+    return v == 1;
+  }
+  static bool tensor(const py::object &o, Tensor &t) {
+    if (!THPVariable_CheckExact(o.ptr())) return false;
+    t = THPVariable_Unpack(o.ptr());
+    return t.layout() == at::kStrided && !t.is_neg() && !t.is_conj() && t.is_contiguous();
+  }
+  static bool number(const py::object &o, double &v) {
+    if (!PyFloat_CheckExact(o.ptr()) && !PyLong_CheckExact(o.ptr())) return false;
+    v = PyFloat_AsDouble(o.ptr());
+    if (v == -1.0 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+    return true;
+  }
+};
+
+py::object quick(const py::object &query, const py::object &key, const py::object &value,
+                 const py::object &seq_lens_k, const py::object &seq_lens_q, bool padded,
+                 const py::object &is_causal, const py::object &scale, const py::object &sigmoid_bias,
+                 const py::object &score_mod) {
+  constexpr int64_t kBwdLimit = (int64_t)2048 << 20;  // _capi._WS_DEFAULT_MB
+  const py::object no = py::none();
+  Tensor q, k, v, sm, lq, lk;
+  if (!g_bound || std::getenv("SIGATTN_EAGER_BINDING") != nullptr ||
+      std::getenv("SIGATTN_BWD_WORKSPACE_MB") != nullptr || !Quick::tensor(query, q) || !Quick::tensor(key, k) ||
+      !Quick::tensor(value, v) || !PyBool_Check(is_causal.ptr()))
+    return no;
+  const at::ScalarType type = q.scalar_type();
+  const at::Device dev = q.device();
+  if (q.dim() != 4 || k.dim() != 4 || k.sizes() != v.sizes() || q.numel() == 0 || k.numel() == 0 ||
+      (type != at::kHalf && type != at::kBFloat16 && type != at::kFloat) || k.scalar_type() != type ||
+      v.scalar_type() != type || !dev.is_cuda() || k.device() != dev || v.device() != dev || !Quick::gfx950(dev.index()))
+    return no;
+  const int64_t B = q.size(0), Tq = q.size(1), Tk = k.size(1), D = q.size(3);
+  if (k.size(0) != B || k.size(2) != q.size(2) || k.size(3) != D || (!padded && Tq != Tk)) return no;
+  if (!score_mod.is_none() &&
+      (!Quick::tensor(score_mod, sm) || sm.scalar_type() != at::kFloat || sm.device() != dev || sm.dim() != 2 ||
+       sm.size(0) != B || sm.size(1) != Tk))
+    return no;
+  double s = 1.0 / std::sqrt((double)D), bias_value = -std::log((double)Tk);
+  if (!scale.is_none() && !Quick::number(scale, s)) return no;
+  const bool own_bias = !sigmoid_bias.is_none();
+  if (own_bias && !Quick::number(sigmoid_bias, bias_value)) return no;
+  const c10::DeviceGuard guard(dev);
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return no;
+  const auto lens = [&](const py::object &o, int64_t T, Tensor &t) {
+    if (o.is_none()) {
+      t = Quick::constant(B, (double)T, at::kInt, dev);
+      return t.defined();
+    }
+    return Quick::tensor(o, t) && t.scalar_type() == at::kInt && t.device() == dev && t.dim() == 1 && t.size(0) == B;
+  };
+  if (padded && (!lens(seq_lens_k, Tk, lk) || !lens(seq_lens_q, Tq, lq))) return no;
+  const Tensor st = Quick::constant(-1, s, at::kFloat, dev);
+  if (!st.defined()) return no;
+  Tensor bias;
+  if (padded && !own_bias) {
+    bias = at::empty({B}, q.options().dtype(at::kFloat).requires_grad(false));
+    check_rc(g_api.default_bias(static_cast<const int32_t *>(lk.data_ptr()), nullptr, B,
+                                static_cast<float *>(bias.data_ptr()), stream),
+             "sigattn_default_bias");
+  } else {
+    bias = Quick::constant(B, bias_value, at::kFloat, dev);
+    if (!bias.defined()) return no;
+  }
+  const auto opt = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
+  return py::cast(SigattnNode::apply(q, k, v, bias, opt(sm), st, opt(lq), opt(lk), is_causal.ptr() == Py_True, kBwdLimit,
+                                     std::nullopt, std::nullopt, 0, 0));
+}
+
 template <class F> void bind_one(F &dst, const py::dict &fns, const char *name) {
   TORCH_CHECK(fns.contains(name), "_sigattn_autograd.bind: missing ", name);
   dst = reinterpret_cast<F>(fns[name].cast<uintptr_t>());
@@ -270,6 +383,7 @@ void bind(const py::dict &fns, const std::vector<int64_t> &two_pass_dims, int64_
   bind_one(api.fwd_decode, fns, "sigattn_fwd_decode");
   bind_one(api.bwd_workspace_bytes, fns, "sigattn_bwd_workspace_bytes");
   bind_one(api.bwd_ws, fns, "sigattn_bwd_ws");
+  bind_one(api.default_bias, fns, "sigattn_default_bias");
   bind_one(api.bwd_split_workspace_bytes, fns, "sigattn_bwd_split_workspace_bytes");
   bind_one(api.bwd_split, fns, "sigattn_bwd_split");
   TORCH_CHECK(dq_ds_rows > 0, "_sigattn_autograd.bind: dq_ds_rows must be positive");
@@ -285,6 +399,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "C++ autograd node of sigmoid_attention / sigmoid_attention_padded over libsigattn";
   m.def("bind", &bind, "Entry point addresses of libsigattn (name -> address), two-pass head dims, "
         "query rows per dQ-from-dS workgroup");
+  m.def("quick", &quick,
+        "sigmoid_attention (padded False) or sigmoid_attention_padded on canonical arguments, or None where the "
+        "Python layer has to take the call",
+        py::arg("query"), py::arg("key"), py::arg("value"), py::arg("seq_lens_k"), py::arg("seq_lens_q"),
+        py::arg("padded"), py::arg("is_causal"), py::arg("scale"), py::arg("sigmoid_bias"), py::arg("score_mod"));
   m.def("attention", &attention,
         "Forward with autograd; arguments are the canonical tensors of _capi._prepare (and _prepare_packed "
         "for the packed layout, with the longest sequences)",

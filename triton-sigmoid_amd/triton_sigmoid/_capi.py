@@ -132,13 +132,16 @@ _EAGER_ENV = "SIGATTN_EAGER_BINDING"
 _AUTOGRAD_FNS = ("sigattn_strerror", "sigattn_fwd_workspace_bytes", "sigattn_fwd_ws",
                  "sigattn_fwd_decode_workspace_bytes", "sigattn_fwd_decode",
                  "sigattn_bwd_workspace_bytes", "sigattn_bwd_ws", "sigattn_bwd_split_workspace_bytes",
-                 "sigattn_bwd_split")
+                 "sigattn_bwd_split", "sigattn_default_bias")
 _autograd = None  # the bound module, or False after a failed import
+# The node's entry for eager calls with canonical arguments (None until the
+# node is bound): the call's result, or None where it does not take it.
+quick = None
 
 
 def autograd_node():
     """The bound C++ autograd module, or None when the Python nodes serve."""
-    global _autograd
+    global _autograd, quick
     if os.environ.get(_EAGER_ENV, "").strip().lower() == "python":
         return None
     if _autograd is None:
@@ -152,7 +155,7 @@ def autograd_node():
             return None
         mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _AUTOGRAD_FNS},
                  list(TWO_PASS_HEAD_DIMS), _DQ_DS_ROWS)
-        _autograd = mod
+        _autograd, quick = mod, mod.quick
     return _autograd or None
 
 

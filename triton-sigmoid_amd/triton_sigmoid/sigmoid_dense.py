@@ -140,6 +140,10 @@ def sigmoid_attention(
     Returns:
         [B, T, H, D] output in the input dtype.
     """
+    if not torch.compiler.is_compiling() and _capi.quick is not None:
+        out = _capi.quick(query, key, value, None, None, False, is_causal, scale, sigmoid_bias, score_mod)
+        if out is not None:
+            return out
     if query.dim() != 4 or key.dim() != 4 or value.dim() != 4:
         raise ValueError("Expected query, key, and value to be 4D tensors")
 

@@ -143,6 +143,11 @@ def sigmoid_attention_padded(
     Returns:
         [B, T_q, H, D] output; rows at or past seq_lens_q[b] are zero.
     """
+    if not torch.compiler.is_compiling() and _capi.quick is not None:
+        out = _capi.quick(query, key, value, seq_lens_k, seq_lens_q, True, is_causal, scale, sigmoid_bias,
+                          score_mod)
+        if out is not None:
+            return out
     if query.dim() != 4 or key.dim() != 4 or value.dim() != 4:
         raise ValueError("Expected query, key, and value to be 4D tensors")
 
