@@ -489,14 +489,14 @@ def test_fp32_values_outside_the_split_match_the_portable_kernels(D, T, causal, 
 # --- D <= 64 forward and dQ: two waves per 32 rows on small grids, one on large ones ---
 
 @pytest.mark.parametrize("D", [16, 32, 64])
-@pytest.mark.parametrize("T", [63, 65, 96, 129])
+@pytest.mark.parametrize("T", [63, 65, 96, 129, 257, 321])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("layout", ["dense", "mod", "padded"])
 def test_wave_pairs_and_single_waves_match_oracle(D, T, causal, layout):
     """17 x 64 (batch, head) pairs are more than four blocks per compute unit
-    (a wave per 32 rows in every kernel); one pair alone is a small grid (two
-    waves per 32 rows).  Both against the oracle, on remainders of 32-, 64-
-    and 128-row blocks."""
+    (a wave per 32 rows, per 64 at D = 64); one pair alone is a small grid (two
+    waves per 32 rows).  Both against the oracle, on remainders of 32-, 64-,
+    128- and 256-row blocks."""
     B, H, dtype = 17, 64, torch.bfloat16
     q, k, v, do = _inputs(B, T, H, D, dtype, seed=T + D)
     g = torch.Generator().manual_seed(T)

@@ -62,12 +62,12 @@ constexpr bool kFwdCausalPairs = SIGATTN_FWD_CAUSAL_PAIRS != 0;
 constexpr int kFwdBhGroup = SIGATTN_FWD_BH_GROUP;
 // Resident workgroups per CU: D = 128 one (128 KB of LDS); D = 64 three (or
 // two with four stages); D = 32 four (32 KB, at most 128 registers per wave).
-template <int D, int WK = 1> constexpr int fwd_occupancy() {
-  return D == 64 ? (fwd_stages<D, WK>() == 3 ? 3 : 2) : (D == 32 ? 4 : 1);
+template <int D, int WK = 1, int NCB = 1> constexpr int fwd_occupancy() {
+  return D == 64 ? (fwd_stages<D, WK>() == 3 && NCB == 1 ? 3 : 2) : (D == 32 ? 4 : 1);
 }
 
 template <typename T, int D, int NWV, int NCB, int WK, bool CAUSAL, bool SCOREMOD>
-__global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK>())) void fwd_mfma_kernel(const KParams p) {
+__global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK, NCB>())) void fwd_mfma_kernel(const KParams p) {
   // NWV waves per workgroup (8: two per SIMD), NCB 32-query column blocks each.
   // WK = 2: the waves form pairs that hold the same queries; wave `wt` of a
   // pair takes block wt of every 64-key tile (one region per tile instead of
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK>())) void fwd_mfma_k
     const auto lq = [&](int i) SIGATTN_INLINE { return p.len_q(i); };
     const auto lk = [&](int i) SIGATTN_INLINE { return p.len_k(i); };
     const WorkItem it = CAUSAL ? WorkOrder::by_level(wg, p.B, p.H, lq, BM, p.nblk, true, p.ncu,
-                                                     fwd_occupancy<D, WK>())
+                                                     fwd_occupancy<D, WK, NCB>())
                                : WorkOrder::by_stream(wg, p.B, p.H, lq, BM, p.nblk, lk);
     b = it.b, h = it.h, qb0 = it.blk;
   } else {
@@ -485,17 +485,17 @@ __global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK>())) void fwd_mfma_k
   }
 }
 
-// Query column blocks per wave: 1 = eight waves of 32 queries (two per SIMD,
-// so each SIMD interleaves two waves' VALU and LDS work); 2 = four waves of
-// 64 queries (every K / Vᵀ operand read feeds two MFMAs).  Measured at the
-// headline shape: 1 is 2-3% faster.
+// Query column blocks per wave at D = 128: 1 = eight waves of 32 queries (two
+// per SIMD, so each SIMD interleaves two waves' VALU and LDS work); 2 = four
+// waves of 64 queries (every K / Vᵀ operand read feeds two MFMAs).  Measured at
+// B=4 L=4096 H=16 causal: 1 is 2-3% faster.
 #ifndef SIGATTN_FWD_NCB
 #define SIGATTN_FWD_NCB 1
 #endif
 
-template <typename T, int D, int NWV, int WK>
+template <typename T, int D, int NWV, int WK, int NCB = SIGATTN_FWD_NCB>
 static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  constexpr int NCB = SIGATTN_FWD_NCB, BM = NWV * 32 * NCB / WK;
+  constexpr int BM = NWV * 32 * NCB / WK;
   KParams p = kp;
   p.nblk = (p.Tq + BM - 1) / BM;
   // Dense causal problems (the kernel's order when not ragged with B <= 64):
@@ -516,9 +516,8 @@ static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStrea
 // D = 128: one workgroup of eight waves per CU (128 KB of LDS).  D = 64: a
 // 3-stage ring of 48 KB, so three workgroups of four waves share a CU (three
 // waves per SIMD, at most 168 VGPRs each) in small work units, which balance
-// better on small or ragged (padded) batches.  Measured against two
-// workgroups per CU with a 4-stage ring: 10-20 % faster dense (c4, c5 shapes)
-// and 5-13 % padded.
+// better on small or ragged (padded) batches than two with a 4-stage ring.  Measured
+// at 10-20 % dense and 5-13 % padded.
 template <typename T, int D>
 static void launch_fwd_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
   // Pairs of waves (WK = 2) where the 128-query blocks number at most one per
@@ -528,6 +527,18 @@ static void launch_fwd_t(const KParams &kp, bool causal, bool scoremod, hipStrea
   // non-causal, 19.8 -> 22.3 causal).
   if constexpr (D <= 64) {
     if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, 1)) return launch_fwd_w<T, D, 4, 2>(kp, causal, scoremod, st);
+  }
+  // 64 queries per wave (D = 64, two workgroups of 256 queries per CU): every
+  // K / Vᵀ operand read from LDS feeds two MFMAs.  With 32 queries the reads
+  // take as many LDS cycles as the MFMAs take matrix cycles, and their energy
+  // lowers the power-limited clock.  Same bits.  bf16 us, 32 -> 64: B=8 T=2048
+  // H=32 339 -> 321 (causal 208 -> 198), B=2 T=8192 H=32 1237 -> 1138 (647 ->
+  // 617), lengths 1487..8192 B=4 H=12 483 -> 449.  The blocks are twice as
+  // long, so it takes two of them per CU (B=4 T=2048 H=16 88 -> 82), four when
+  // their lengths differ by the causal mask (two per CU: 49.8 / 49.6).
+  if constexpr (D == 64) {
+    if (kp.rsplit <= 1 && (int64_t)kp.B * kp.H * ((kp.Tq + 255) / 256) >= (causal ? 4 : 2) * (int64_t)kp.ncu)
+      return launch_fwd_w<T, D, 4, 1, 2>(kp, causal, scoremod, st);
   }
   launch_fwd_w<T, D, (D <= 64 ? 4 : 8) / SIGATTN_FWD_NCB, 1>(kp, causal, scoremod, st);
 }
