@@ -498,13 +498,26 @@ template <int D, int WK> constexpr int fwd_f32_occupancy() {
 }
 template <int D, int WK> constexpr int bwd_f32_occupancy() { return D < 128 && WK * D <= 128 ? 2 : 1; }
 
-// (batch, head) and row block of a workgroup, causal ones with the most work
-// first (forward and dQ: the last block).
-template <int WK> __device__ __forceinline__ Item item_of(const KParams &p, int wg, bool last_first) {
+// (batch, head) and row block of a workgroup, those with the most work first:
+// ragged batches in WorkOrder's order (ROWS_Q: the rows are queries), causal
+// dense ones from the last query or first key block.  occ: workgroups per CU.
+// Ragged, forward + backward, us, in index order / WorkOrder's: padded B=4
+// T=3000 H=8 D=64 1350 / 971, packed causal B=8 T=1500 H=8 D=128 949 / 726.
+// (Dense blocks of one head on one XCD, as the 16-bit kernels have them: B=2
+// T=1024 H=8 D=64 145 -> 152.)
+template <int WK, bool CAUSAL, bool ROWS_Q>
+__device__ __forceinline__ Item item_of(const KParams &p, int wg, int occ) {
   constexpr int RB = 32 * FW / WK;
+  if (p.ragged() && p.B <= 64) {
+    const auto rows = [&](int i) SIGATTN_INLINE { return ROWS_Q ? p.len_q(i) : p.len_k(i); };
+    const auto stream = [&](int i) SIGATTN_INLINE { return ROWS_Q ? p.len_k(i) : p.len_q(i); };
+    const WorkItem it = CAUSAL ? WorkOrder::by_level(wg, p.B, p.H, rows, RB, p.nblk, ROWS_Q, p.ncu, occ)
+                               : WorkOrder::by_stream(wg, p.B, p.H, rows, RB, p.nblk, stream);
+    return Item{it.b, it.h, it.blk * RB, it.blk * RB + RB};
+  }
   const int BH = p.B * p.H, bh = wg % BH;
   int blk = wg / BH;
-  if (last_first) blk = p.nblk - 1 - blk;
+  if (CAUSAL && ROWS_Q) blk = p.nblk - 1 - blk;
   return Item{bh / p.H, bh % p.H, blk * RB, blk * RB + RB};
 }
 
@@ -519,7 +532,7 @@ __global__ __launch_bounds__(64 * FW, (fwd_f32_occupancy<D, WK>())) void fwd_f32
 
   const int wg = gap_prologue<4>(p, lds);  // packed layouts: leading gap-zeroing workgroups
   if (wg < 0) return;
-  const Item it = item_of<WK>(p, wg, CAUSAL);
+  const Item it = item_of<WK, CAUSAL, true>(p, wg, fwd_f32_occupancy<D, WK>());
   const int b = it.b, h = it.h;
   const int Lq = p.len_q(b), Lk = p.len_k(b);
   const bool half = p.half_head(D);
@@ -598,7 +611,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dq_f32_
 
   const int wg = gap_prologue<4>(p, lds);  // packed layouts: leading gap-zeroing workgroups
   if (wg < 0) return;
-  const Item it = item_of<WK>(p, wg, CAUSAL);
+  const Item it = item_of<WK, CAUSAL, true>(p, wg, bwd_f32_occupancy<D, WK>());
   const int b = it.b, h = it.h;
   const int Lq = p.len_q(b), Lk = p.len_k(b);
   const bool half = p.half_head(D);
@@ -675,7 +688,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
   __shared__ __attribute__((aligned(16))) float lds[lds_floats<D, WK>()];
   uint16_t *tiles = (uint16_t *)lds;
 
-  const Item it = item_of<WK>(p, blockIdx.x, false);  // causal: low key blocks (the most work) first
+  const Item it = item_of<WK, CAUSAL, false>(p, blockIdx.x, bwd_f32_occupancy<D, WK>());
   const int b = it.b, h = it.h;
   const int Lq = p.len_q(b), Lk = p.len_k(b);
   const bool half = p.half_head(D);
