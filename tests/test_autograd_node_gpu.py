@@ -12,6 +12,8 @@ import math
 
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import triton_sigmoid as ts
 from helpers import randn
@@ -276,3 +278,42 @@ def test_quick_entry_leaves_errors_and_overrides_to_the_python_layer(monkeypatch
         monkeypatch.setenv(name, value)
         assert _capi.quick(q, q, q, None, None, False, False, None, None, None) is None
         monkeypatch.delenv(name)
+
+
+class _Seen(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Dispatched(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("mode", [_Seen, _Dispatched])
+def test_quick_entry_leaves_calls_under_a_mode_to_the_python_layer(mode):
+    q = torch.randn((1, 24, 2, 32), device=DEV, dtype=torch.float16)
+    want = ts.sigmoid_attention(q, q, q)
+    with mode():
+        assert _capi.quick(q, q, q, None, None, False, False, None, None, None) is None
+        got = ts.sigmoid_attention(q, q, q)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("binding", ["quick", "layer"])
+def test_training_after_the_same_shape_under_inference_mode(monkeypatch, binding):
+    """The kept scale, bias and length constants made by a call under inference
+    mode serve a later call that saves them for backward."""
+    q0 = torch.randn((5, 23 if binding == "quick" else 29, 1, 16), device=DEV, dtype=torch.float16)
+    ts.sigmoid_attention(q0[:1], q0[:1], q0[:1])  # binds the node
+    if binding == "layer":
+        monkeypatch.setattr(_capi, "quick", None)
+        monkeypatch.setattr(_capi, "autograd_node", lambda node=_capi.autograd_node(): node)
+    for fn in (ts.sigmoid_attention, ts.sigmoid_attention_padded):
+        with torch.inference_mode():
+            want = fn(q0, q0, q0, scale=0.37)
+        q = q0.clone().requires_grad_(True)
+        o = fn(q, q0, q0, scale=0.37)
+        assert torch.equal(o.detach(), want)
+        o.sum().backward()
+        assert torch.isfinite(q.grad).all()

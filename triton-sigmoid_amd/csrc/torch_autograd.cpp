@@ -266,7 +266,9 @@ Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor
 // layer's per-call checks and conversions (about 6 of 12 us of host time, which
 // is what a small call takes): exact torch.Tensors, contiguous, one gfx950
 // device, matching shapes, plain numbers, no environment overrides, no stream
-// capture.  Everything else -- and so every error -- is None, and the Python
+// capture, no function or dispatch mode or functorch transform (which see the
+// Python layer's operators, and would put their own tensors among the kept
+// constants).  Everything else -- and so every error -- is None, and the Python
 // layer takes the call.
 struct Quick {
   // Constants [n] on a device, as _capi.device_constant keeps them: made by a
@@ -280,6 +282,7 @@ struct Quick {
     const auto it = kept->find(key);
     if (it != kept->end()) return it->second;
     if (kept->size() >= kMax || std::isnan(value)) return Tensor();
+    const c10::InferenceMode normal(false);  // kept for calls that save it for backward too
     const auto opt = at::TensorOptions().dtype(type);
     const Tensor t = (n < 0 ? at::full({}, value, opt) : at::full({n}, value, opt)).to(dev);
     kept->emplace(key, t);
@@ -296,6 +299,10 @@ struct Quick {
       known[dev].store(v, std::memory_order_relaxed);
     }
     return v == 1;
+  }
+  static bool observed() {
+    return at::impl::torch_function_mode_enabled() || c10::impl::dispatch_mode_enabled() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
   }
   static bool tensor(const py::object &o, Tensor &t) {
     if (!THPVariable_CheckExact(o.ptr())) return false;
@@ -320,7 +327,7 @@ py::object quick(const py::object &query, const py::object &key, const py::objec
   constexpr int64_t kBwdLimit = (int64_t)2048 << 20;  // _capi._WS_DEFAULT_MB
   const py::object no = py::none();
   Tensor q, k, v, sm, lq, lk;
-  if (!g_bound || std::getenv("SIGATTN_EAGER_BINDING") != nullptr ||
+  if (!g_bound || Quick::observed() || std::getenv("SIGATTN_EAGER_BINDING") != nullptr ||
       std::getenv("SIGATTN_BWD_WORKSPACE_MB") != nullptr || !Quick::tensor(query, q) || !Quick::tensor(key, k) ||
       !Quick::tensor(value, v) || !PyBool_Check(is_causal.ptr()))
     return no;

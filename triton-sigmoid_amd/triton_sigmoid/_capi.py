@@ -569,6 +569,7 @@ def device_constant(shape, value, dtype: torch.dtype, device) -> torch.Tensor:
             # the current stream (freed by torch's allocator in that stream's
             # order) takes its place.
             return torch.full(shape, value, dtype=dtype, device=dev)
-        t = torch.full(shape, value, dtype=dtype).to(dev)
+        with torch.inference_mode(False):  # a later call may save it for backward
+            t = torch.full(shape, value, dtype=dtype).to(dev)
         _CONSTANTS[key] = t
     return t
