@@ -163,11 +163,15 @@ def test_decode_long_cache_sum_of_halves():
 
 
 @pytest.mark.parametrize("B,H,Tq,Tk,D,packed,mod", [
-    (8, 16, 1, 2100, 64, False, False),    # 9 chunks of 256, the last short
+    (8, 16, 1, 2100, 64, False, False),    # chunks of at least 256 keys
     (10, 13, 3, 2111, 128, False, True),   # units not a multiple of the workgroup's four
-    (8, 16, 32, 8200, 64, False, True),    # all 32 query rows; chunks of 1088
+    (8, 16, 32, 8200, 64, False, True),    # all 32 query rows
     (9, 16, 2, 3001, 128, True, True),     # packed rows
     (16, 128, 2, 300, 64, False, False),   # one chunk per (batch, head): no partials
+    (64, 16, 1, 700, 64, False, False),    # a batch per lane, 2 rows of partials each
+    (65, 16, 1, 700, 64, False, False),    # one more: chunks of one length for all
+    (12, 16, 32, 12000, 64, False, False), # keys for one round of waves, not for two
+    (3, 16, 1, 30000, 128, False, True),   # ... and long sequences
 ])
 def test_decode_wave_per_chunk_matches_the_general_path(B, H, Tq, Tk, D, packed, mod):
     """sigattn_fwd_decode's plan (a wave per chunk) against sigattn_fwd_ws and

@@ -98,7 +98,7 @@ bool use_f32_mfma(const sigattn_problem *p, const void *const *ptrs, int nptr) {
 // decode shapes, targets from 256 to 2048 workgroups run within noise of each
 // other; 512 keeps the partials small.
 struct SplitPlan {
-  int nsplit = 0, chunk = 0, unit_waves = 4;
+  int nsplit = 0, chunk = 0, unit_waves = 4, rows = 0, round_rows = 0;
 };
 
 #ifndef SIGATTN_SPLIT_TARGET
@@ -136,6 +136,15 @@ SplitPlan splitkv_plan(const sigattn_problem *p, bool mfma) {
 // 4 / 8 / 16 / 32, us: B=16 H=32 D=128 Tk=8192 full 319 / 323 / 366 / 412,
 // lengths 1186..8192 199 / 195 / 198 / 197, B=32 H=32 D=64 Tq=4 Tk=4096 214 /
 // 167 / 171 / 176, B=12 H=12 D=64 Tq=8 lengths 800..6001 49 / 37 / 41 / 41.
+// The chunks of one length for all sequences behind these figures leave ragged
+// caches' last chunks short, so the device cuts batches of up to a lane per
+// sequence by their lengths into two rounds of waves, or one where two would
+// need chunks below `least`.  Us, one length / cut: B=16 H=32 D=128 lengths
+// 1186..8192 196 / 175, B=4 H=16 up to 32768 129 / 113, B=8 H=16 Tq=32 up to
+// 16000 121 / 107, B=32 H=32 D=64 Tq=4 up to 4097 125 / 107; full caches as
+// before (330 / 329, 174 / 177), the one draw of five with chunks that happened
+// to fit 247 / 253.
+constexpr int64_t kDecodeCutBatch = 64, kDecodeCutKeys = 1 << 20;
 constexpr int64_t kDecodeChunk = 256, kDecodeMinWaves = 4, kDecodeWaves = 8;
 SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
   SplitPlan sp = splitkv_plan(p, mfma);
@@ -152,11 +161,20 @@ SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
   sp.nsplit = (int)cdiv(p->Tk, chunk);
   sp.chunk = (int)chunk;
   sp.unit_waves = 1;
+  if (sp.nsplit > 1 && p->B <= kDecodeCutBatch && p->Tk < kDecodeCutKeys) {
+    const int64_t round = kDecodeMinWaves * cus / p->H;
+    sp.rows = (int)(kDecodeWaves / kDecodeMinWaves * round);
+    if (sp.rows < 2 * p->B || sp.rows > sp.nsplit * p->B) sp.rows = (int)(sp.nsplit * p->B);
+    if (round >= 2 * p->B && round < sp.rows) sp.round_rows = (int)round;
+    sp.chunk = (int)least;
+  }
   return sp;
 }
 
 int64_t splitkv_workspace_bytes(const sigattn_problem *p, const SplitPlan &sp) {
-  return sp.nsplit > 1 ? (int64_t)sp.nsplit * p->B * p->H * p->Tq * p->D * (int64_t)sizeof(float) : 0;
+  const int64_t cut = sp.rows > 0 ? 2 * p->B * (int64_t)sizeof(int32_t) : 0;
+  const int64_t rows = sp.rows > 0 ? sp.rows : (int64_t)sp.nsplit * p->B;
+  return sp.nsplit > 1 ? rows * p->H * p->Tq * p->D * (int64_t)sizeof(float) + cut : 0;
 }
 
 bool is_ragged(const sigattn_problem *p) {
@@ -599,6 +617,8 @@ static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t
     k.nsplit = sp.nsplit;
     k.chunk = sp.chunk;
     k.unit_waves = sp.unit_waves;
+    k.rows = sp.rows;
+    k.round_rows = sp.round_rows;
     sigattn::launch_fwd_splitkv(k, p->dtype, (int)p->D, p->score_mod != nullptr, st);
   } else if (mfma) {
     sigattn::launch_fwd_mfma(k, p->dtype, mfma_head_dim(p), p->causal != 0, p->score_mod != nullptr, st);

@@ -99,7 +99,10 @@ struct KParams {
   // Split-KV forward: keys cut into nsplit chunks of `chunk` keys; fp32
   // partials [nsplit, B, H, Tq, D] in ws when nsplit > 1.
   // unit_waves: waves that share one (batch, head, chunk), 4 or 1.
-  int nsplit, chunk, unit_waves;
+  // rows > 0 (unit_waves = 1): the partials are [rows, H, Tq, D] and the device
+  // cuts the batch into at most `rows` chunks of at least `chunk` keys;
+  // round_rows > 0: as many as the GPU runs at a time, at least 2 B.
+  int nsplit, chunk, unit_waves, rows, round_rows;
   float *ws;
   // Two-pass backward: dS in the I/O dtype as 32x32 tiles (see DsLayout),
   // written by the dK/dV kernel and read by the dQ-from-dS kernel.

@@ -92,9 +92,58 @@ hipError_t splitkv_scratch(float **ptr) {
 //     H=32 D=64 Tq=4 Tk=4096 216 -> 166 us (6.9 TB/s without the calls' other
 //     launches); one-wave workgroups on the heads of one XCD took 348, 364 and
 //     214 us, two-wave ones 317, 317 and 191.
+//     Ragged caches would leave such units uneven, so the device cuts the
+//     sequences (WaveUnits): p.rows chunks in all, of about equal length.
 // A wave's K and V blocks have two stages each; the K stage is refilled as
 // soon as S is computed and the V stage after the output product, so three of
 // the four blocks are in flight at any time.
+// The cut of a batch (B <= 64, keys < 2^20 each) into at most p.rows chunks of
+// equal length or nearly so, from the lengths on the device; every wave
+// of the chunk kernel computes it alike (in the reduction too it took 10 us more
+// at 4096 output rows: B=32 H=32 D=64 Tq=4 Tk=4096 178 -> 190 us), and leaves
+// each sequence's first row and chunk length for the reduction.  The longest chunk C is the
+// smallest of 64 candidates, one a lane, from total / rows (at least p.chunk)
+// upwards that gives at most p.rows chunks: sum ceil(L / C) <= total / C + B,
+// and the last candidate is 2.9 times the first, so one fits where B <= rows / 2.
+// A sequence of L keys then has n = ceil(L / C) chunks of ceil(L / n) keys.
+struct WaveUnits {
+  int len, n;  // of sequence `lane`
+
+  // ceil(L / C) by the half-integer quotient, which is off every integer by
+  // 1 / 2C, more than its rounding error for L < 2^20.
+  static __device__ __forceinline__ int ceil_div(int L, float rc) {
+    return L > 0 ? (int)(((float)L - 0.5f) * rc) + 1 : 0;
+  }
+  __device__ __forceinline__ WaveUnits(const KParams &p, int lane) {
+    len = lane < p.B ? p.len_k(lane) : 0;
+    int total = 0;  // < 2^26
+    for (int i = 0; i < p.B; ++i) total += __builtin_amdgcn_readlane(len, i);
+    // Too few keys for p.rows chunks of p.chunk: one round of the GPU's waves
+    // rather than a second, nearly empty one.
+    int rows = p.rows;
+    if (total < rows * (int64_t)p.chunk && p.round_rows > 0 && total >= p.round_rows * (int64_t)p.chunk)
+      rows = p.round_rows;
+    const int c0 = (max((total + rows - 1) / rows, p.chunk) + 31) / 32;  // in blocks of 32 keys
+    const int c = 32 * (c0 + (c0 * lane * lane + 2047) / 2048);
+    float rc = 1.0f / (float)c;
+    int count = 0;
+    for (int i = 0; i < p.B; ++i) count += ceil_div(__builtin_amdgcn_readlane(len, i), rc);
+    const int j = __builtin_ctzll(__ballot(count <= rows) | (1ull << 63));
+    rc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rc), j));
+    n = ceil_div(len, rc);
+  }
+  // Keys of one chunk of sequence b; its last chunks may be empty.
+  __device__ __forceinline__ int keys(int b) const {
+    const int L = __builtin_amdgcn_readlane(len, b), m = __builtin_amdgcn_readlane(n, b);
+    return ((L + m - 1) / max(m, 1) + 31) & ~31;
+  }
+};
+
+// (first row, keys of a chunk) of every sequence with keys, after the partials.
+__device__ __forceinline__ int2 *cut_of(const KParams &p, int D) {
+  return (int2 *)(p.ws + (int64_t)p.rows * p.H * p.Tq * D);
+}
+
 template <typename T, int D, int WPU, bool SCOREMOD, bool DIRECT>
 __global__ __launch_bounds__(256, 1) void fwd_splitkv_kernel(const KParams p) {
   constexpr int NW = 4;
@@ -112,17 +161,35 @@ __global__ __launch_bounds__(256, 1) void fwd_splitkv_kernel(const KParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
-  const int NS = p.nsplit, C = p.chunk;
-  int s, b, h;
-  if (WPU == 1) {
+  const int NS = p.nsplit;
+  int s, b, h, C = p.chunk;
+  int64_t row;  // of the partials: (chunk, batch), or the unit's of WaveUnits
+  if (WPU == 1 && !DIRECT && p.rows > 0) {
+    const unsigned u = blockIdx.x * NW + w, H = p.H, r = u / H;
+    if (r >= (unsigned)p.rows) return;
+    h = (int)(u - r * H);
+    row = r;
+    const WaveUnits wu(p, lane);
+    s = (int)r;
+    for (b = 0; b < p.B; ++b) {
+      const int n = __builtin_amdgcn_readlane(wu.n, b);
+      if (s < n) break;
+      s -= n;
+    }
+    if (b == p.B) return;
+    C = wu.keys(b);
+    if (s == 0 && h == 0 && lane == 0) cut_of(p, D)[b] = make_int2((int)r, C);
+  } else if (WPU == 1) {
     const unsigned u = blockIdx.x * NW + w, H = p.H, r = u / H;  // units fit 31 bits (sigattn_check)
     if (u >= H * (unsigned)p.B * (unsigned)NS) return;
     h = (int)(u - r * H);
     s = (int)(r % (unsigned)NS);
     b = (int)(r / (unsigned)NS);
+    row = (int64_t)s * p.B + b;
   } else {
     const int bh = blockIdx.x / NS;
     s = blockIdx.x % NS, b = bh / p.H, h = bh % p.H;
+    row = (int64_t)s * p.B + b;
   }
   const int wu = WPU == 1 ? 0 : w;  // the wave's place in its unit
   const int Lq = p.len_q(b), Lk = p.len_k(b);
@@ -242,7 +309,7 @@ __global__ __launch_bounds__(256, 1) void fwd_splitkv_kernel(const KParams p) {
   }
 
   float *ws_row = nullptr;
-  if (!DIRECT) ws_row = p.ws + (((int64_t)s * p.B + b) * p.H + h) * p.Tq * D;
+  if (!DIRECT) ws_row = p.ws + (row * p.H + h) * p.Tq * D;
   uint16_t *Ob = (uint16_t *)p.out + qoff;
   if constexpr (WPU == 1) {
     const bool valid = l32 < Lq;
@@ -314,9 +381,15 @@ __global__ __launch_bounds__(256) void fwd_splitkv_reduce_kernel(const KParams p
   if (q >= p.q_rows_out(Lq)) return;
   f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
   if (q < Lq) {
-    const int nvs = (Lk + p.chunk - 1) / p.chunk;
-    const int64_t step = (int64_t)p.B * p.H * p.Tq * D;
-    const float *src = p.ws + ((int64_t)bh * p.Tq + q) * D + 4 * c;
+    int C = p.chunk;
+    int64_t row = b, rows = p.B;  // first partial of (b, h), and rows from one to the next
+    if (p.rows > 0 && Lk > 0) {
+      const int2 cut = cut_of(p, D)[b];
+      row = cut.x, C = cut.y, rows = 1;
+    }
+    const int nvs = (Lk + C - 1) / C;
+    const int64_t step = rows * p.H * p.Tq * D;
+    const float *src = p.ws + ((row * p.H + h) * p.Tq + q) * D + 4 * c;
 #pragma unroll 4
     for (int s = g; s < nvs; s += NG) v += *(const f32x4 *)(src + s * step);
   }
@@ -331,7 +404,7 @@ __global__ __launch_bounds__(256) void fwd_splitkv_reduce_kernel(const KParams p
 
 template <typename T, int D, int WPU>
 static void launch_chunks(const KParams &p, bool scoremod, hipStream_t st) {
-  const int64_t units = (int64_t)p.B * p.H * p.nsplit;
+  const int64_t units = p.rows > 0 ? (int64_t)p.rows * p.H : (int64_t)p.B * p.H * p.nsplit;
   const dim3 grid((unsigned)(WPU == 1 ? (units + 3) / 4 : units)), block(256);
   if (p.nsplit == 1) {
     if (scoremod) fwd_splitkv_kernel<T, D, WPU, true, true><<<grid, block, 0, st>>>(p);
