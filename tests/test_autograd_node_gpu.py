@@ -317,3 +317,27 @@ def test_training_after_the_same_shape_under_inference_mode(monkeypatch, binding
         assert torch.equal(o.detach(), want)
         o.sum().backward()
         assert torch.isfinite(q.grad).all()
+
+
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("which", ["scale", "sigmoid_bias"])
+def test_quick_entry_gives_nan_for_a_nan_scale_or_bias(monkeypatch, padded, which):
+    """A NaN scale or bias is not any constant kept from an earlier call: O and
+    the gradients are NaN, as the Python layer's, and so they are again after
+    another finite call."""
+    B, T = 7, 19
+    q = torch.randn((B, T, 1, 16), device=DEV, dtype=torch.float16)
+    fn = ts.sigmoid_attention_padded if padded else ts.sigmoid_attention
+
+    def run(**kw):
+        ins = [q.clone().requires_grad_(True) for _ in range(3)]
+        o = fn(*ins, **kw)
+        return (o.detach(), *torch.autograd.grad(o, ins, torch.ones_like(o)))
+
+    for value in (0.125, -3.5):
+        assert all(torch.isfinite(t).all() for t in run(**{which: value}))
+        for _ in range(2):
+            got = run(**{which: math.nan})
+            assert all(torch.isnan(t).all() for t in got)
+    monkeypatch.setattr(_capi, "quick", None)
+    assert all(torch.isnan(t).all() for t in run(**{which: math.nan}))

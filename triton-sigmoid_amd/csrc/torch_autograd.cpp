@@ -275,13 +275,14 @@ struct Quick {
   // blocking copy, at most kMax, never freed (a queued kernel may read one).
   static constexpr size_t kMax = 256;
   static Tensor constant(int64_t n, double value, at::ScalarType type, const at::Device &dev) {
+    if (std::isnan(value)) return Tensor();  // has no place in the map's order: it would match any kept value
     static std::mutex mu;
     static auto *kept = new std::map<std::tuple<int, int64_t, double, int>, Tensor>;  // outlives every thread
     const std::tuple<int, int64_t, double, int> key(dev.index(), n, value, (int)type);
     std::lock_guard<std::mutex> lock(mu);
     const auto it = kept->find(key);
     if (it != kept->end()) return it->second;
-    if (kept->size() >= kMax || std::isnan(value)) return Tensor();
+    if (kept->size() >= kMax) return Tensor();
     const c10::InferenceMode normal(false);  // kept for calls that save it for backward too
     const auto opt = at::TensorOptions().dtype(type);
     const Tensor t = (n < 0 ? at::full({}, value, opt) : at::full({n}, value, opt)).to(dev);
