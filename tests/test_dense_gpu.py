@@ -486,6 +486,72 @@ def test_fp32_values_outside_the_split_match_the_portable_kernels(D, T, causal, 
         torch.testing.assert_close(got[fine], want[fine], rtol=0, atol=2 ** -24 * 64 * top)
 
 
+def _fp32_and_portable(ins, mod, causal):
+    """O, dQ, dK, dV of the fp32 kernels and of the portable ones (heads D + 1
+    floats apart, so most rows start off 16 bytes), bias -2."""
+    B, T, H, D = ins[0].shape
+    lib = _capi.load_library()
+    bias = torch.full((B,), -2.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    both = []
+    for pad in (0, 1):
+        i = [torch.nn.functional.pad(t, (0, pad))[..., :D] for t in ins]
+        o = [torch.nn.functional.pad(torch.full_like(t, 7.0), (0, pad))[..., :D] for t in ins]
+        pr = _capi._problem(*i[:3], bias, mod, scale, None, None, causal)
+        assert lib.sigattn_fwd(ctypes.byref(pr), o[0].data_ptr(), stream) == 0
+        assert lib.sigattn_bwd(ctypes.byref(pr), i[3].data_ptr(), *(t.data_ptr() for t in o[1:]), stream) == 0
+        torch.cuda.synchronize()
+        both.append(o)
+    return both
+
+
+@pytest.mark.parametrize("D,B,H,T", [(32, 2, 3, 96), (64, 2, 3, 320), (64, 4, 64, 257), (128, 2, 3, 161)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kind", ["q", "k", "q-denormal", "do-v", "v-do", "do-k", "do-q", "one-key", "one-query",
+                                  "probability"])
+def test_fp32_tiny_operands_of_ordinary_results_match_the_portable_kernels(D, B, H, T, causal, kind):
+    """Operands too small for three bf16 parts against large ones, so that the
+    scores, dP or the results are of a size that shows nothing of it."""
+    q, k, v, do = _inputs(B, T, H, D, torch.float32, seed=T + D)
+    mod = None
+    if kind == "q":
+        q, k = q * 1e-35, k * 1e35
+    elif kind == "k":
+        q, k = q * 1e35, k * 1e-35
+    elif kind == "q-denormal":
+        q, k = q * 1e-38, k * 1e36
+    elif kind == "do-v":
+        do, v = do * 1e-36, v * 1e36
+    elif kind == "v-do":
+        do, v = do * 1e36, v * 1e-36
+    elif kind == "do-k":
+        do, q, k = do * 1e-36, q * 1e-12, k * 1e12
+    elif kind == "do-q":
+        do, q, k = do * 1e-36, q * 1e12, k * 1e-12
+    elif kind == "probability":  # P and dS, not the inputs, are tiny
+        q, k, v, do, mod = q * 1e-13, k * 1e12, v * 1e30, do * 1e-30, torch.full((B, T), -83.0, device=DEV)
+    elif kind == "one-key":  # a single streamed (dQ) or stationary (dK, dV) row
+        k[0, T - 2, 1] *= 1e-35
+        q[0, :, 1, :3] *= 1e35
+        k[0, :T - 2, 1, :3] = 0.0
+        k[0, T - 1:, 1, :3] = 0.0
+        q[0, :, 1, 3:] = 0.0
+    else:
+        q[0, T - 1, 1] *= 1e-35
+        k[0, :, 1, :3] *= 1e35
+        q[0, :T - 1, 1, :3] = 0.0
+        k[0, :, 1, 3:] = 0.0
+    got, want = _fp32_and_portable((q, k, v, do), mod, causal)
+    for name, x, y in zip(("O", "dQ", "dK", "dV"), got, want):
+        assert torch.isfinite(y).all(), name
+        # fp32 sums of up to T and D terms in two orders: a few roundings of a head's largest value.
+        # Scores near -83 are 2^7 as exponents of two, whose last bit is 2^-17: two of those in P.
+        top = y.abs().amax(dim=(1, 3), keepdim=True)
+        bound = 2 ** -24 * 64 + (2 ** -16 if kind == "probability" else 0)
+        assert torch.all((x - y).abs() <= bound * top), (name, ((x - y).abs() / top).max().item())
+
+
 # --- D <= 64 forward and dQ: two waves per 32 rows on small grids, one on large ones ---
 
 @pytest.mark.parametrize("D", [16, 32, 64])

@@ -19,10 +19,20 @@
 // D/2 of 64: 2.7 times fewer matrix cycles.
 //
 // Values that have no such split (infinities, NaN, magnitudes above bf16's
-// largest) become NaN there, and magnitudes below about 2^-110 lose their
-// lower parts to the flush of 16-bit denormals.  So a workgroup that ends with
-// a NaN or with a nonzero value below 2^-96 computes its rows again with
-// v_mfma_f32_32x32x2_f32 (the *_full functions) and stores those.
+// largest) become NaN there, and magnitudes below 2^-110 lose lower bits:
+// bf16's denormals, which the matrix instruction keeps, end at 2^-133, so a
+// value is off by up to 2^-134 and a product by that times the other factor.
+// A workgroup whose results may show it computes its rows again with
+// v_mfma_f32_32x32x2_f32 (the *_full functions) and stores those.  With every
+// input at most M in magnitude, S is off by 2^-126·M at most (nothing, for the
+// sigmoid, unless scale or M is huge), dP as much, and a result by 2^-112·M²
+// for each of its terms and roundings of its own: the rows are computed again
+// where a result is NaN or below 2^-88·(M / 2^7)² (M at least 2^7), or where
+// M >= 2^60 or the scale >= 2^32.  A zero is taken for one, unless M > 2^24:
+// it may stand for less than 2^-110 a term.  Finding M costs one instruction
+// for two split values: forward, dQ, dK/dV, us, B=2 T=1999 H=8 D=64 causal
+// 73.7, 90.1, 133.7 -> 75.0, 91.4, 133.0, B=2 T=4096 H=16 D=128 causal 857,
+// 1079, 1614 -> 841, 1123, 1668.
 #include <type_traits>
 
 #include "common.h"
@@ -334,6 +344,33 @@ __device__ __forceinline__ void split8(f32x4 x, f32x4 y, u32x4 (&o)[3]) {
   }
 }
 
+// The largest magnitude of the inputs that a thread split.
+struct SplitRange {
+  float top = 0.0f;
+  __device__ __forceinline__ void see(f32x4 x) {
+    // fmaxf would canonicalise every operand first.
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(x.x), "v"(x.y));
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(x.z), "v"(x.w));
+  }
+  // The first parts of a stationary row, after the loop: looked at where they
+  // are split, they hold up the first tile's loads (0.8 us of a 16 us kernel).
+  template <int N> __device__ __forceinline__ void see(const u32x4 (&part)[N]) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 m = {0, 0};
+#pragma unroll
+    for (int s = 0; s < N; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, part[s][e] & 0x7fff7fffu));
+    const uint32_t most = m.x > m.y ? m.x : m.y;
+    top = fmaxf(top, __builtin_bit_cast(float, most << 16));
+  }
+  // Results need more than the look at 2^-88.
+  __device__ __forceinline__ bool wide(float scale) const {
+    return top > 0x1p7f || !(__builtin_fabsf(scale) < 0x1p32f);
+  }
+};
+
 // The lane's stationary row as B operands of the three parts (k = 16s + 8hi + j);
 // zeros when !ok and, for head_dim 16 in the D = 32 kernels, past column 16.
 template <int D>
@@ -374,9 +411,10 @@ template <int D, int TR> struct SplitTiles {
       r[i][1] = in ? *(const f32x4 *)(src + 4) : z;
     }
   }
-  __device__ __forceinline__ void store(uint16_t *lds) const {
+  __device__ __forceinline__ void store(uint16_t *lds, SplitRange &rg) const {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
+      rg.see(r[i][0]), rg.see(r[i][1]);
       const int ch = threadIdx.x + 64 * FW * i;
       const int off = toff<D>(ch % CH / (D / 8), 8 * (ch % (D / 8)));
       u32x4 o[3];
@@ -439,17 +477,32 @@ __device__ __forceinline__ void row3(f32x16 (&acc)[D / 32], const uint16_t *t, c
   }
 }
 
-// True where a value has no place in the split's range: NaN, or nonzero below 2^-96.
-template <int N> __device__ __forceinline__ bool out_of_range(const f32x16 (&acc)[N]) {
+// True where a result is NaN, or below `least` and not zero (or zero too).
+template <int N> __device__ __forceinline__ bool in_doubt(const f32x16 (&acc)[N], float least, bool zeros) {
   bool bad = false;
 #pragma unroll
   for (int db = 0; db < N; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const float a = __builtin_fabsf(acc[db][i]);
-      bad |= !(a >= 0x1p-96f || a == 0.0f);
+      bad |= !(a >= least || (a == 0.0f && !zeros));
     }
   return bad;
+}
+
+// The smallest result that is not in doubt, and whether zeros are, for the
+// workgroup's largest input; false where that is out of range.  All threads
+// call it; no wave uses `lds` any more once all have arrived here.
+__device__ __forceinline__ bool doubt_below(const SplitRange &rg, float *lds, float &least, bool &zeros) {
+  uint32_t *most = (uint32_t *)lds;
+  if (threadIdx.x == 0) *most = 0;
+  __syncthreads();
+  atomicMax(most, __builtin_bit_cast(uint32_t, rg.top));
+  __syncthreads();
+  const float m = __builtin_bit_cast(float, *most);
+  const float r = m * 0x1p-7f > 1.0f ? m * 0x1p-7f : 1.0f;
+  least = 0x1p-88f * r * r, zeros = m > 0x1p24f;
+  return m < 0x1p60f;
 }
 
 // Adds the accumulators of a row group's waves into its first wave, in wave
@@ -552,6 +605,7 @@ __global__ __launch_bounds__(64 * FW, (fwd_f32_occupancy<D, WK>())) void fwd_f32
   const float scale = *p.scale, bias = p.bias[b];
   const float nsl = -scale * kLog2e, nbl = -bias * kLog2e;
 
+  SplitRange rg;
   u32x4 qf[3][NKS];
   load_split_row<D>(qf, (const float *)p.q + qoff + (int64_t)myq * p.sq_t, hi, myq < Lq, half);
   f32x16 acc[NDB];
@@ -569,7 +623,7 @@ __global__ __launch_bounds__(64 * FW, (fwd_f32_occupancy<D, WK>())) void fwd_f32
   if (nsteps > 0) load(0);
   for (int t = 0; t < nsteps; ++t) {
     __syncthreads();  // every read of step t - 1 is done
-    st.store(tiles);
+    st.store(tiles, rg);
     if (SCOREMOD && tid < TR) sC[tid] = creg;
     if (t + 1 < nsteps) load(t + 1);
     __syncthreads();
@@ -592,9 +646,15 @@ __global__ __launch_bounds__(64 * FW, (fwd_f32_occupancy<D, WK>())) void fwd_f32
     row3<D, Tiles::PART>(acc, Tiles::part(tiles, 1, 0), to, 2 * wt, pr);
   }
   add_waves<NDB, WK>(acc, lds, w, lane);
-  if (__syncthreads_or(wt == 0 && myq < Lq && out_of_range(acc))) {
-    fwd_full<D, CAUSAL, SCOREMOD>(p, it, lds);
-    return;
+  if (wt == 0) rg.see(qf[0]);
+  if (__syncthreads_or((wt == 0 && myq < Lq && in_doubt(acc, 0x1p-88f, false)) || rg.wide(scale))) {
+    float least;
+    bool zeros;
+    const bool fits = doubt_below(rg, lds, least, zeros) && __builtin_fabsf(scale) < 0x1p32f;
+    if (__syncthreads_or(!fits || (wt == 0 && myq < Lq && in_doubt(acc, least, zeros)))) {
+      fwd_full<D, CAUSAL, SCOREMOD>(p, it, lds);
+      return;
+    }
   }
   if (wt == 0 && myq < p.q_rows_out(Lq))
     store_row<D>((float *)p.out + qoff + (int64_t)myq * p.sq_t, acc, 1.0f, myq < Lq, hi, half);
@@ -630,6 +690,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dq_f32_
   const float scale = *p.scale, bias = p.bias[b];
   const float nsl = -scale * kLog2e, nbl = -bias * kLog2e;
 
+  SplitRange rg;
   u32x4 qf[3][NKS], of[3][NKS];
   load_split_row<D>(qf, (const float *)p.q + qoff + (int64_t)myq * p.sq_t, hi, myq < Lq, half);
   load_split_row<D>(of, (const float *)p.dout + qoff + (int64_t)myq * p.sq_t, hi, myq < Lq, half);
@@ -648,7 +709,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dq_f32_
   if (nsteps > 0) load(0);
   for (int t = 0; t < nsteps; ++t) {
     __syncthreads();
-    st.store(tiles);
+    st.store(tiles, rg);
     if (SCOREMOD && tid < TR) sC[tid] = creg;
     if (t + 1 < nsteps) load(t + 1);
     __syncthreads();
@@ -672,9 +733,15 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dq_f32_
     row3<D, Tiles::PART>(acc, tiles, to, 2 * wt, ds);
   }
   add_waves<NDB, WK>(acc, lds, w, lane);
-  if (__syncthreads_or(wt == 0 && myq < Lq && out_of_range(acc))) {
-    dq_full<D, CAUSAL, SCOREMOD>(p, it, lds);
-    return;
+  if (wt == 0) rg.see(qf[0]), rg.see(of[0]);
+  if (__syncthreads_or((wt == 0 && myq < Lq && in_doubt(acc, 0x1p-88f, false)) || rg.wide(scale))) {
+    float least;
+    bool zeros;
+    const bool fits = doubt_below(rg, lds, least, zeros) && __builtin_fabsf(scale) < 0x1p32f;
+    if (__syncthreads_or(!fits || (wt == 0 && myq < Lq && in_doubt(acc, least, zeros)))) {
+      dq_full<D, CAUSAL, SCOREMOD>(p, it, lds);
+      return;
+    }
   }
   if (wt == 0 && myq < p.q_rows_out(Lq))
     store_row<D>((float *)p.dq + qoff + (int64_t)myq * p.sq_t, acc, scale, myq < Lq, hi, half);
@@ -708,6 +775,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
   float nc = -bias * kLog2e;
   if (SCOREMOD) nc = kok ? -(bias + p.score_mod[p.mod_base(b) + myk]) * kLog2e : 0.0f;
 
+  SplitRange rg;
   u32x4 kf[3][NKS], vf[3][NKS];
   load_split_row<D>(kf, (const float *)p.k + koff + (int64_t)myk * p.sk_t, hi, kok, half);
   load_split_row<D>(vf, (const float *)p.v + koff + (int64_t)myk * p.sk_t, hi, kok, half);
@@ -721,7 +789,7 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
   if (nsteps > 0) load(0);
   for (int t = 0; t < nsteps; ++t) {
     __syncthreads();
-    st.store(tiles);
+    st.store(tiles, rg);
     if (t + 1 < nsteps) load(t + 1);
     __syncthreads();
     const int m0 = mstart + t * TR + FB * wt;
@@ -753,9 +821,16 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
   }
   add_waves<NDB, WK>(dva, lds, w, lane);
   add_waves<NDB, WK>(dka, lds, w, lane);
-  if (__syncthreads_or(wt == 0 && kok && (out_of_range(dva) || out_of_range(dka)))) {
-    dkdv_full<D, CAUSAL, SCOREMOD>(p, it, lds);
-    return;
+  if (wt == 0) rg.see(kf[0]), rg.see(vf[0]);
+  if (__syncthreads_or((wt == 0 && kok && (in_doubt(dva, 0x1p-88f, false) || in_doubt(dka, 0x1p-88f, false))) ||
+                       rg.wide(scale))) {
+    float least;
+    bool zeros;
+    const bool fits = doubt_below(rg, lds, least, zeros) && __builtin_fabsf(scale) < 0x1p32f;
+    if (__syncthreads_or(!fits || (wt == 0 && kok && (in_doubt(dva, least, zeros) || in_doubt(dka, least, zeros))))) {
+      dkdv_full<D, CAUSAL, SCOREMOD>(p, it, lds);
+      return;
+    }
   }
   if (wt == 0 && myk < p.k_rows_out(Lk)) {
     store_row<D>((float *)p.dk + koff + (int64_t)myk * p.sk_t, dka, scale, kok, hi, half);
