@@ -160,7 +160,8 @@ int sigattn_fwd_ws(const sigattn_problem *p, void *out, void *workspace, size_t 
  * sigattn_fwd_decode_workspace_bytes(p) bytes of partials; every other
  * problem runs, and asks for, exactly what sigattn_fwd_ws does.  Deterministic,
  * and equal to sigattn_fwd_ws within fp32 summation order.  With workspace
- * NULL it is sigattn_fwd; a workspace smaller than the partials returns
+ * NULL a problem that needs partials runs as in sigattn_fwd; one chunk per
+ * (batch, head) needs none.  A workspace smaller than the partials returns
  * SIGATTN_ERR_WORKSPACE.
  */
 size_t sigattn_fwd_decode_workspace_bytes(const sigattn_problem *p);

@@ -219,3 +219,37 @@ def test_decode_wave_per_chunk_matches_the_general_path(B, H, Tq, Tk, D, packed,
                                  scale=np.float32(1 / math.sqrt(D)), bias=np.full(1, -3.0), score_mod=ms,
                                  with_bwd=False)
         assert_close_to_oracle(outs[0][b:b + 1, :, heads], want, torch.bfloat16, f"sequence {b}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Tq,Tk,D", [(16, 128, 2, 300, 64), (16, 128, 1, 257, 128),  # enough (batch, head) pairs
+                                         (8, 128, 32, 1000, 64)])                        # one chunk of 32 Tq keys
+@pytest.mark.parametrize("mod", [False, True])
+def test_decode_wave_per_pair_is_what_callers_without_a_workspace_get(dtype, B, H, Tq, Tk, D, mod):
+    """One chunk per (batch, head) needs no partials: the public entry and a call
+    without a workspace run the same kernel as one that is handed some memory."""
+    lib = _capi.load_library()
+    g = torch.Generator().manual_seed(Tk + D)
+    lens = torch.randint(1, Tk + 1, (B,), generator=g)
+    lens[0], lens[1], lens[2] = Tk, 0, 33
+    q = randn((B, Tq, H, D), dtype, DEV, g)
+    k, v = (randn((B, Tk, H, D), dtype, DEV, g) for _ in range(2))
+    sm = torch.randn((B, Tk), generator=g).to(DEV) if mod else None
+    bias = torch.full((B,), -3.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    sq = torch.full((B,), Tq, dtype=torch.int32, device=DEV)
+    sk = lens.to(DEV, torch.int32)
+    pr = _capi._problem(q, k, v, bias, sm, scale, sq, sk, False)
+    assert lib.sigattn_fwd_decode_workspace_bytes(ctypes.byref(pr)) == 0
+    stream = torch.cuda.current_stream().cuda_stream
+    some = torch.zeros(256, dtype=torch.uint8, device=DEV)
+    want, got, other = (torch.full_like(q, float("nan")) for _ in range(3))
+    assert lib.sigattn_fwd_decode(ctypes.byref(pr), want.data_ptr(), some.data_ptr(), 0, stream) == 0
+    assert lib.sigattn_fwd_decode(ctypes.byref(pr), got.data_ptr(), None, 0, stream) == 0
+    assert lib.sigattn_fwd(ctypes.byref(pr), other.data_ptr(), stream) == 0
+    api = ts.sigmoid_attention_padded(q, k, v, sk, sq, sigmoid_bias=-3.0, score_mod=sm)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(api, want)
+    # The shared form adds in another order: one rounding of the largest value.
+    torch.testing.assert_close(want, other, atol=2 ** -7 * other.abs().max().item(), rtol=0)
+    assert not torch.equal(want, other)

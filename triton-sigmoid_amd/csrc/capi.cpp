@@ -573,9 +573,9 @@ static int fwd_impl(const sigattn_problem *p, void *out, void *workspace, size_t
   const void *ptrs[4] = {p->q, p->k, p->v, out};
   const bool mfma = use_mfma(p, ptrs, 4);
   SplitPlan sp = splitkv_plan(p, mfma);
-  if (decode && workspace != nullptr) {
+  if (decode) {
     const SplitPlan dp = decode_plan(p, mfma);
-    if (dp.nsplit > 0) sp = dp;
+    if (dp.nsplit == 1 || (dp.nsplit > 1 && workspace != nullptr)) sp = dp;
   }
   if (sp.nsplit > 1 && static_scratch) {
     if ((size_t)splitkv_workspace_bytes(p, sp) > sigattn::kSplitScratchBytes) return SIGATTN_ERR_SCRATCH;
