@@ -253,3 +253,33 @@ def test_decode_wave_per_pair_is_what_callers_without_a_workspace_get(dtype, B, 
     # The shared form adds in another order: one rounding of the largest value.
     torch.testing.assert_close(want, other, atol=2 ** -7 * other.abs().max().item(), rtol=0)
     assert not torch.equal(want, other)
+
+
+def _plan_bytes(B, H, Tq, Tk, D):
+    """Workspace of the decode plan and of the shared form."""
+    lib = _capi.load_library()
+    q = torch.empty((B, Tq, H, D), dtype=torch.bfloat16, device=DEV)
+    k = torch.empty((B, Tk, H, D), dtype=torch.bfloat16, device=DEV)
+    n = torch.empty((B,), dtype=torch.int32, device=DEV)
+    f = torch.empty((B,), dtype=torch.float32, device=DEV)
+    pr = _capi._problem(q, k, k, f, None, f[0], n, n, False)
+    return tuple(int(fn(ctypes.byref(pr))) for fn in (lib.sigattn_fwd_decode_workspace_bytes,
+                                                      lib.sigattn_fwd_workspace_bytes))
+
+
+@pytest.mark.parametrize("B,H,Tq,Tk,D", [(24, 32, 16, 581, 64), (48, 32, 1, 469, 64), (80, 16, 4, 378, 64),
+                                         (64, 8, 2, 672, 64), (128, 4, 32, 2614, 64), (16, 32, 1, 299, 128)])
+def test_short_caches_of_many_pairs_need_no_partials(B, H, Tq, Tk, D):
+    """From 512 (batch, head) pairs on the shared form writes O itself; caches
+    that are read in less time than the partials take keep it."""
+    assert _plan_bytes(B, H, Tq, Tk, D) == (0, 0)
+
+
+@pytest.mark.parametrize("B,H,Tq,Tk,D,packed,mod", [
+    (64, 16, 1, 2100, 64, False, True),   # a sequence per lane
+    (65, 16, 1, 2100, 64, False, True),   # one more: chunks of one length for all
+    (72, 8, 2, 2600, 128, True, False),   # ... five of them, packed rows
+    (80, 4, 1, 6000, 64, False, False),
+])
+def test_decode_large_batches_match_the_general_path(B, H, Tq, Tk, D, packed, mod):
+    test_decode_wave_per_chunk_matches_the_general_path(B, H, Tq, Tk, D, packed, mod)

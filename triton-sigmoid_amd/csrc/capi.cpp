@@ -142,10 +142,16 @@ SplitPlan splitkv_plan(const sigattn_problem *p, bool mfma) {
 // need chunks below `least`.  Us, one length / cut: B=16 H=32 D=128 lengths
 // 1186..8192 196 / 175, B=4 H=16 up to 32768 129 / 113, B=8 H=16 Tq=32 up to
 // 16000 121 / 107, B=32 H=32 D=64 Tq=4 up to 4097 125 / 107; full caches as
-// before (330 / 329, 174 / 177), the one draw of five with chunks that happened
-// to fit 247 / 253.
+// before (330 / 329, 174 / 177).
+// Where the shared form writes O itself (512 pairs), the partials and their
+// second launch have to be paid for by what the reads gain, about a fifth:
+// kDecodeBytes of K and V and kDecodeRowBytes for each row of O.  Us, shared /
+// this: B=24 H=32 D=64 Tq=16 Tk=581 23.5 / 42.4, B=48 H=32 D=64 Tk=469 32.5 /
+// 42.3, B=32 H=24 D=128 Tq=2 Tk=950 (373 MB) 73.5 / 71.3, B=96 H=16 D=64
+// Tk=1059 (416 MB) 84.2 / 69.8.
 constexpr int64_t kDecodeCutBatch = 64, kDecodeCutKeys = 1 << 20;
 constexpr int64_t kDecodeChunk = 256, kDecodeMinWaves = 4, kDecodeWaves = 8;
+constexpr int64_t kDecodeBytes = 340 << 20, kDecodeRowBytes = 34 << 10;
 SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
   SplitPlan sp = splitkv_plan(p, mfma);
   if (sp.nsplit == 0) return sp;
@@ -157,8 +163,10 @@ SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
   if (cus <= 0 || pairs * most < kDecodeMinWaves * cus) return SplitPlan{};
   int64_t n = cdiv(kDecodeWaves * cus, pairs);
   if (n > most) n = most;
-  const int64_t chunk = cdiv(cdiv(p->Tk, n), 64) * 64;
+  const int64_t chunk = cdiv(cdiv(p->Tk, n), 64) * 64, bytes = 4 * p->D * pairs * p->Tk;
+  const bool shared_writes = sp.nsplit == 1;
   sp.nsplit = (int)cdiv(p->Tk, chunk);
+  if (sp.nsplit > 1 && shared_writes && bytes < kDecodeBytes + kDecodeRowBytes * pairs * p->Tq) return SplitPlan{};
   sp.chunk = (int)chunk;
   sp.unit_waves = 1;
   if (sp.nsplit > 1 && p->B <= kDecodeCutBatch && p->Tk < kDecodeCutKeys) {
