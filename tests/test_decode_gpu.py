@@ -275,6 +275,15 @@ def test_short_caches_of_many_pairs_need_no_partials(B, H, Tq, Tk, D):
     assert _plan_bytes(B, H, Tq, Tk, D) == (0, 0)
 
 
+@pytest.mark.parametrize("B,H,Tq,Tk,D,chunks", [(65, 16, 1, 2100, 64, 3), (80, 16, 1, 8192, 128, 3),
+                                                (72, 8, 2, 2600, 128, 5), (80, 4, 1, 6000, 64, 7),
+                                                (256, 1, 1, 20000, 64, 7), (70, 8, 1, 3000, 64, 5)])
+def test_batches_of_more_than_a_lane_each_take_an_odd_number_of_chunks(B, H, Tq, Tk, D, chunks):
+    """An even number would put the last, short chunks of all sequences on the
+    same XCDs."""
+    assert _plan_bytes(B, H, Tq, Tk, D)[0] == chunks * B * H * Tq * D * 4
+
+
 @pytest.mark.parametrize("B,H,Tq,Tk,D,packed,mod", [
     (64, 16, 1, 2100, 64, False, True),   # a sequence per lane
     (65, 16, 1, 2100, 64, False, True),   # one more: chunks of one length for all

@@ -143,6 +143,11 @@ SplitPlan splitkv_plan(const sigattn_problem *p, bool mfma) {
 // 1186..8192 196 / 175, B=4 H=16 up to 32768 129 / 113, B=8 H=16 Tq=32 up to
 // 16000 121 / 107, B=32 H=32 D=64 Tq=4 up to 4097 125 / 107; full caches as
 // before (330 / 329, 174 / 177).
+// Larger batches keep one length, with an odd number of chunks: workgroups go
+// to the XCDs in turn, and an even number would put every sequence's last,
+// short or empty chunk on the same ones.  Us, even / odd: B=72 H=16 D=128
+// lengths 512..8192 2 / 3 chunks 617 / 451 (shared 529), full 774 / 743; B=72
+// H=8 lengths 256..4096 4 / 5 chunks 163 / 119 (shared 142).
 // Where the shared form writes O itself (512 pairs), the partials and their
 // second launch have to be paid for by what the reads gain, about a fifth:
 // kDecodeBytes of K and V and kDecodeRowBytes for each row of O.  Us, shared /
@@ -162,8 +167,11 @@ SplitPlan decode_plan(const sigattn_problem *p, bool mfma) {
   const int64_t most = cdiv(p->Tk, least);
   if (cus <= 0 || pairs * most < kDecodeMinWaves * cus) return SplitPlan{};
   int64_t n = cdiv(kDecodeWaves * cus, pairs);
+  const auto chunk_of = [&](int64_t m) { return cdiv(cdiv(p->Tk, m), 64) * 64; };
+  if (p->B > kDecodeCutBatch && n > 1)
+    for (n = n <= 4 ? n | 1 : (n - 1) | 1; n + 2 <= most && cdiv(p->Tk, chunk_of(n)) % 2 == 0;) n += 2;
   if (n > most) n = most;
-  const int64_t chunk = cdiv(cdiv(p->Tk, n), 64) * 64, bytes = 4 * p->D * pairs * p->Tk;
+  const int64_t chunk = chunk_of(n), bytes = 4 * p->D * pairs * p->Tk;
   const bool shared_writes = sp.nsplit == 1;
   sp.nsplit = (int)cdiv(p->Tk, chunk);
   if (sp.nsplit > 1 && shared_writes && bytes < kDecodeBytes + kDecodeRowBytes * pairs * p->Tq) return SplitPlan{};
