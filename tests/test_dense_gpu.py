@@ -592,3 +592,29 @@ def test_wave_pairs_and_single_waves_match_oracle(D, T, causal, layout):
             assert_close_to_oracle(x[b:b + 1, :n, h:h + 1], want, dtype, f"{name}, large grid")
             assert_close_to_oracle(y[:, :n], want, dtype, f"{name}, alone")
             assert torch.all(x[b, n:] == 0) and torch.all(y[:, n:] == 0)
+
+
+@pytest.mark.parametrize("T", [961, 1000, 1023, 1024])  # remainders of 32-, 64-, 128- and 256-row blocks
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("layout", ["dense", "mod", "padded"])
+def test_wide_waves_match_oracle(T, causal, layout):
+    """Four blocks of 256 queries per compute unit (eight of padded ones) run 64
+    queries per wave at D = 64: O of a few sequences and heads."""
+    B, H, D, dtype = 32 if layout == "padded" else 16, 16, 64, torch.bfloat16
+    q, k, v, _ = _inputs(B, T, H, D, dtype, seed=T)
+    g = torch.Generator().manual_seed(T)
+    mod = torch.randn((B, T), generator=g).to(DEV) if layout == "mod" else None
+    lens = torch.full((B,), T, dtype=torch.int32)
+    if layout == "padded":
+        lens[1:] = torch.randint(1, T + 1, (B - 1,), generator=g, dtype=torch.int32)
+        n = lens.to(DEV)
+        o = ts.sigmoid_attention_padded(q, k, v, n, n, is_causal=causal, sigmoid_bias=-2.0)
+    else:
+        o = ts.sigmoid_attention(q, k, v, is_causal=causal, sigmoid_bias=-2.0, score_mod=mod)
+    for b, h in ((0, 0), (3, H - 1), (B - 1, 7)):
+        n = int(lens[b])
+        one = [t[b:b + 1, :n, h:h + 1] for t in (q, k, v)]
+        want, _ = oracle_fwd_bwd(*one, None, scale=np.float32(1.0 / math.sqrt(D)), bias=np.full(1, -2.0), causal=causal,
+                                 score_mod=None if mod is None else mod[b:b + 1], with_bwd=False)
+        assert_close_to_oracle(o[b:b + 1, :n, h:h + 1], want, dtype, "O")
+        assert torch.all(o[b, n:] == 0)

@@ -513,6 +513,29 @@ static void launch_fwd_w(const KParams &kp, bool causal, bool scoremod, hipStrea
   }
 }
 
+// 64 queries per wave (D = 64, two workgroups of 256 queries per CU): every
+// K / Vᵀ operand read from LDS feeds two MFMAs.  With 32 queries the reads take
+// as many LDS cycles as the MFMAs take matrix cycles, and their energy lowers
+// the power-limited clock.  Same bits.  bf16 us, 32 -> 64: B=8 T=2048 H=32 339
+// -> 321 (causal 208 -> 198), B=2 T=8192 H=32 1237 -> 1138 (647 -> 617),
+// lengths 1487..8192 B=4 H=12 483 -> 449.  The blocks are twice as long, which
+// costs more than that where
+//   * a sequence has few of them, or ends in half of one (T=513 to 845 up to 33 %
+//     slower, T=1025 23 %, T=1152 3-20 %; from 2048 rows on half a block is 6 %);
+//   * the grid is small.  Times of 64 over 32, by 256-query blocks per CU f:
+//     dense f = 2.06..2.5 1.06-1.12, 3.06..3.5 1.01-1.04, but 2.0, 2.53..3.0 and
+//     3.56..4.0 0.92-0.96 -- the blocks of 128 of an odd round fill CUs that
+//     the long blocks leave half empty -- and f > 4 0.92-1.02; causal f = 4..5
+//     0.97-1.02, f = 8 0.92-0.97; lengths T/16..T f = 4..5 0.91-1.39, 6..7
+//     0.94-1.03 from T = 2000 on (T = 1000 1.09, causal), f = 8 0.93-1.02.
+static bool wide_waves(const KParams &p, bool causal) {
+  const int64_t n = (p.Tq + 127) / 128, blocks = (int64_t)p.B * p.H * ((p.Tq + 255) / 256), cus = p.ncu;
+  if (cus <= 0 || n < 8 || (n % 2 != 0 && n < 16)) return false;
+  if (p.ragged()) return blocks >= (n < 16 ? 8 : 6) * cus;
+  if (blocks >= 4 * cus) return true;
+  return !causal && blocks >= 2 * cus && (2 * blocks + cus - 1) / cus % 2 == 0;
+}
+
 // D = 128: one workgroup of eight waves per CU (128 KB of LDS).  D = 64: a
 // 3-stage ring of 48 KB, so three workgroups of four waves share a CU (three
 // waves per SIMD, at most 168 VGPRs each) in small work units, which balance
@@ -528,17 +551,8 @@ static void launch_fwd_t(const KParams &kp, bool causal, bool scoremod, hipStrea
   if constexpr (D <= 64) {
     if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, 1)) return launch_fwd_w<T, D, 4, 2>(kp, causal, scoremod, st);
   }
-  // 64 queries per wave (D = 64, two workgroups of 256 queries per CU): every
-  // K / Vᵀ operand read from LDS feeds two MFMAs.  With 32 queries the reads
-  // take as many LDS cycles as the MFMAs take matrix cycles, and their energy
-  // lowers the power-limited clock.  Same bits.  bf16 us, 32 -> 64: B=8 T=2048
-  // H=32 339 -> 321 (causal 208 -> 198), B=2 T=8192 H=32 1237 -> 1138 (647 ->
-  // 617), lengths 1487..8192 B=4 H=12 483 -> 449.  The blocks are twice as
-  // long, so it takes two of them per CU (B=4 T=2048 H=16 88 -> 82), four when
-  // their lengths differ by the causal mask (two per CU: 49.8 / 49.6).
   if constexpr (D == 64) {
-    if (kp.rsplit <= 1 && (int64_t)kp.B * kp.H * ((kp.Tq + 255) / 256) >= (causal ? 4 : 2) * (int64_t)kp.ncu)
-      return launch_fwd_w<T, D, 4, 1, 2>(kp, causal, scoremod, st);
+    if (kp.rsplit <= 1 && wide_waves(kp, causal)) return launch_fwd_w<T, D, 4, 1, 2>(kp, causal, scoremod, st);
   }
   launch_fwd_w<T, D, (D <= 64 ? 4 : 8) / SIGATTN_FWD_NCB, 1>(kp, causal, scoremod, st);
 }
