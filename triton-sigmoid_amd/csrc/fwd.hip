@@ -543,13 +543,13 @@ static bool wide_waves(const KParams &p, bool causal) {
 // at 10-20 % dense and 5-13 % padded.
 template <typename T, int D>
 static void launch_fwd_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  // Pairs of waves (WK = 2) where the 128-query blocks number at most one per
-  // CU: half of every block's chain (fp16 B=2 T=1024 H=8 D=64, 128 blocks: call
-  // 16.8 -> 12.2 us).  Beyond, a tile per region leaves its copy one region of
-  // time and the fourth stage the third workgroup (512 blocks 27.6 -> 31.2 us
-  // non-causal, 19.8 -> 22.3 causal).
+  // Pairs of waves (WK = 2, fwd_wave_pairs): half of every block's chain (fp16
+  // B=2 T=1024 H=8 D=64, 128 blocks: call 16.8 -> 12.2 us).  Beyond one block
+  // per CU, a tile per region leaves its copy one region of time and the fourth
+  // stage the third workgroup (512 blocks 27.6 -> 31.2 us non-causal, 19.8 ->
+  // 22.3 causal).
   if constexpr (D <= 64) {
-    if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, 1)) return launch_fwd_w<T, D, 4, 2>(kp, causal, scoremod, st);
+    if (kp.rsplit <= 1 && fwd_wave_pairs(kp)) return launch_fwd_w<T, D, 4, 2>(kp, causal, scoremod, st);
   }
   if constexpr (D == 64) {
     if (kp.rsplit <= 1 && wide_waves(kp, causal)) return launch_fwd_w<T, D, 4, 1, 2>(kp, causal, scoremod, st);

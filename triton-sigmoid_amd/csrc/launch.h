@@ -16,16 +16,24 @@ constexpr int kF32 = 2;
 // without a GPU).  Defined with the C ABI.
 int device_compute_units();
 
-// Rows per workgroup and resident workgroups per CU of the MFMA forward and
-// of the recompute backward's kernels (D in {64, 128}); the range split of
-// small dense grids (KParams::rsplit) sizes itself from them.
-// At most `per_cu` 128-row blocks per compute unit: where the D <= 64 forward
-// and dQ kernels let two waves share each 32 rows (half the chain per workgroup,
-// twice the workgroups).
+// Where the D <= 64 forward and dQ kernels let two waves share each 32 rows
+// (half the chain per workgroup, twice the workgroups and tile copies), by
+// their 128-row blocks per compute unit.  Forward: at most one; half of one
+// where a sequence is one block (T = 100, causal, us, one wave / two: half a
+// block per CU 0.92-0.96 of the time, 0.8 to one 1.05-1.12).
+inline bool fwd_wave_pairs(const KParams &p) {
+  const int64_t n = (p.Tq + 127) / 128;
+  return (n == 1 ? 2 : 1) * n * p.B * p.H <= p.ncu;
+}
+
+// At most `per_cu` 128-row blocks per compute unit: where dQ does.
 inline bool wave_pairs(const KParams &p, int rows, int per_cu) {
   return (int64_t)p.B * p.H * ((rows + 127) / 128) <= per_cu * (int64_t)p.ncu;
 }
 
+// Rows per workgroup and resident workgroups per CU of the MFMA forward and
+// of the recompute backward's kernels (D in {64, 128}); the range split of
+// small dense grids (KParams::rsplit) sizes itself from them.
 int fwd_rows_per_workgroup(int D);
 int fwd_workgroups_per_cu(int D);
 int bwd_dq_rows_per_workgroup();
