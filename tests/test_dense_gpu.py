@@ -618,3 +618,36 @@ def test_wide_waves_match_oracle(T, causal, layout):
                                  score_mod=None if mod is None else mod[b:b + 1], with_bwd=False)
         assert_close_to_oracle(o[b:b + 1, :n, h:h + 1], want, dtype, "O")
         assert torch.all(o[b, n:] == 0)
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("B,H,T", [(10, 20, 63), (10, 10, 129), (5, 13, 321)])  # 200, 200 and 195 blocks of 128 rows
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("with_mod", [False, True])
+def test_dq_wave_pairs_of_dense_grids_match_oracle(D, B, H, T, causal, with_mod):
+    """Dense grids of up to one 128-row block per compute unit that do not fit
+    the one-launch backward's single workgroup per unit run dQ in pairs of
+    waves: two of the heads against the oracle, and the same bits apart."""
+    dtype = torch.bfloat16
+    q, k, v, do = _inputs(B, T, H, D, dtype, seed=T + D)
+    g = torch.Generator().manual_seed(T)
+    mod = torch.randn((B, T), generator=g).to(DEV) if with_mod else None
+    bias = torch.full((B,), -2.0, device=DEV)
+    scale = torch.tensor(1 / math.sqrt(D), device=DEV)
+    lib = _capi.load_library()
+    pr = _capi._problem(q, k, v, bias, mod, scale, None, None, causal)
+    one = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    two = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.sigattn_bwd(ctypes.byref(pr), do.data_ptr(), *(t.data_ptr() for t in one), stream) == 0
+    assert lib.sigattn_bwd_dq(ctypes.byref(pr), do.data_ptr(), two[0].data_ptr(), stream) == 0
+    assert lib.sigattn_bwd_dkdv(ctypes.byref(pr), do.data_ptr(), two[1].data_ptr(), two[2].data_ptr(), stream) == 0
+    torch.cuda.synchronize()
+    for a, b in zip(one, two):
+        assert torch.equal(a, b)
+    for b, h in ((0, H - 1), (B - 1, 1)):
+        ins = [t[b:b + 1, :, h:h + 1] for t in (q, k, v, do)]
+        _, grads = oracle_fwd_bwd(*ins, scale=np.float32(1.0 / math.sqrt(D)), bias=np.full(1, -2.0), causal=causal,
+                                  score_mod=None if mod is None else mod[b:b + 1])
+        for name, x, want in zip(("dQ", "dK", "dV"), one, grads):
+            assert_close_to_oracle(x[b:b + 1, :, h:h + 1], want, dtype, name)

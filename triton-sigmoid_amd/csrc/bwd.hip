@@ -641,20 +641,20 @@ __global__ __launch_bounds__(256, (D <= 64 ? 2 : 1)) void bwd_dkdv_kernel(const 
 }
 
 // The recompute backward's two kernels in one launch: the first nkv workgroups
-// run dK/dV items, the rest dQ items, in pairs of waves as launch_bwd_dq_mfma
+// run dK/dV items, the rest dQ items, WK waves to 32 rows as launch_bwd_dq_mfma
 // runs these grids.  On grids within one workgroup per CU the two halves share
 // the GPU instead of each leaving half of it idle; on causal ones of several,
 // the short dQ items run beside the dK/dV kernel's last ones.  The bodies are
 // the kernels' own, so results are bit-identical to the two launches.  They
 // share their LDS, and two workgroups fit a CU.
-template <typename T, int D, bool CAUSAL, bool SCOREMOD>
-__global__ __launch_bounds__(256, 2) void bwd_fused_kernel(const KParams pq, const KParams pk, int nkv) {
+template <typename T, int D, int WK, bool CAUSAL, bool SCOREMOD>
+__global__ __launch_bounds__(256, WK) void bwd_fused_kernel(const KParams pq, const KParams pk, int nkv) {
   __shared__ __attribute__((aligned(16))) union {
     DqLds<D, SCOREMOD> dq;
     DkdvLds<D> dkdv;
   } lds;
   if ((int)blockIdx.x < nkv) bwd_dkdv_body<T, D, CAUSAL, SCOREMOD, false>(pk, blockIdx.x, lds.dkdv);
-  else bwd_dq_body<T, D, 2, CAUSAL, SCOREMOD>(pq, (int)blockIdx.x - nkv, lds.dq);
+  else bwd_dq_body<T, D, WK, CAUSAL, SCOREMOD>(pq, (int)blockIdx.x - nkv, lds.dq);
 }
 
 // ---------------------------------------------------------------------------
@@ -1330,17 +1330,18 @@ static void bwd_dq_w(const KParams &kp, bool causal, bool sm, hipStream_t st) {
   });
 }
 
-// Pairs of waves (WK = 2, D <= 64) halve the longest item's chain for twice the
-// tile copies.  Causal and ragged grids end with their longest items, so they
-// gain up to four 128-row blocks per CU (fp16 causal B=8 Lmax=2048 H=8 D=64,
-// lengths 641..2048, 1024 blocks: 50.7 -> 41.5 us); equal items gain only where
-// they leave CUs idle (B=4 T=1500 H=16 D=64 non-causal, 768 blocks, forward +
-// backward: 211 -> 216 us).
+// Pairs of waves (WK = 2, D <= 64, dq_wave_pairs) halve the longest item's chain
+// for twice the tile copies (fp16 causal B=8 Lmax=2048 H=8 D=64, lengths
+// 641..2048, 1024 blocks: 50.7 -> 41.5 us; B=4 T=1500 H=16 D=64 non-causal, 768
+// blocks, forward + backward: 211 -> 216 us, which keeps one wave).
+static bool dq_pairs(const KParams &p, bool causal) {
+  return dq_wave_pairs((int64_t)p.B * p.H, p.Tq, p.Tk, causal, p.ragged(), p.ncu);
+}
+
 template <typename T, int D>
 static void bwd_dq_t(const KParams &kp, bool causal, bool sm, hipStream_t st) {
   if constexpr (D <= 64) {
-    if (kp.rsplit <= 1 && wave_pairs(kp, kp.Tq, causal || kp.ragged() ? 4 : 1))
-      return bwd_dq_w<T, D, 2>(kp, causal, sm, st);
+    if (kp.rsplit <= 1 && dq_pairs(kp, causal)) return bwd_dq_w<T, D, 2>(kp, causal, sm, st);
   }
   bwd_dq_w<T, D, 1>(kp, causal, sm, st);
 }
@@ -1470,19 +1471,25 @@ void launch_bwd_fused_mfma(const KParams &kp, int dtype, int D, bool causal, boo
     constexpr int DD = decltype(d)::value;
     if constexpr (DD <= 64) {
       KParams pq = kp, pk = kp;
-      pq.nblk = (kp.Tq + 63) / 64;
+      const bool pairs = dq_pairs(kp, causal);
+      pq.nblk = pairs ? (kp.Tq + 63) / 64 : (kp.Tq + 127) / 128;
       pk.nblk = (kp.Tk + 127) / 128;
       pq.rsplit = pk.rsplit = 1;
       pq.ngap[0] = pq.ngap[1] = pk.ngap[0] = pk.ngap[1] = 0;  // no packed layouts: no gap rows
       const int nkv = pk.nblk * kp.B * kp.H;
       const dim3 grid((unsigned)(nkv + pq.nblk * kp.B * kp.H));
-      if (causal) {
-        if (sm) bwd_fused_kernel<T, DD, true, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
-        else bwd_fused_kernel<T, DD, true, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
-      } else {
-        if (sm) bwd_fused_kernel<T, DD, false, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
-        else bwd_fused_kernel<T, DD, false, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
-      }
+      const auto launch = [&](auto wk) {
+        constexpr int WK = decltype(wk)::value;
+        if (causal) {
+          if (sm) bwd_fused_kernel<T, DD, WK, true, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
+          else bwd_fused_kernel<T, DD, WK, true, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
+        } else if constexpr (WK == 1) {  // a workgroup per CU
+          if (sm) bwd_fused_kernel<T, DD, WK, false, true><<<grid, 256, 0, st>>>(pq, pk, nkv);
+          else bwd_fused_kernel<T, DD, WK, false, false><<<grid, 256, 0, st>>>(pq, pk, nkv);
+        }
+      };
+      if (pairs) launch(std::integral_constant<int, 2>{});
+      else launch(std::integral_constant<int, 1>{});
     }
   });
 }

@@ -203,9 +203,9 @@ bool is_ragged(const sigattn_problem *p) {
 //   * the problem is dense and the two grids (128 rows per workgroup)
 //     together need at most one workgroup per CU: apart, each would leave the
 //     CUs the other needs idle; or
-//   * it is causal and not packed, with at most six such workgroups per CU
-//     (and no more dQ ones than launch_bwd_dq_mfma runs in pairs of waves, the
-//     one-launch kernel's form): each kernel alone ends with few CUs busy.
+//   * it is causal and not packed, its dQ runs in pairs of waves
+//     (dq_wave_pairs), and the two take at most six such workgroups per CU:
+//     each kernel alone ends with few CUs busy.
 //     Forward + backward, us, apart / one launch: B=1 T=8000 H=8 D=64, four
 //     per CU, 398 / 371; B=2 T=2048 H=16 D=32, four, 99.4 / 89.7; B=4 T=1500
 //     H=16 D=64, six, 138.6 / 133.8; B=8 T=2048 H=8 D=64, eight, 223 / 234 (dQ
@@ -217,7 +217,8 @@ bool fuse_backward(const sigattn_problem *p) {
   const int64_t ndq = p->B * p->H * cdiv(p->Tq, 128), nkv = p->B * p->H * cdiv(p->Tk, 128);
   if (cus <= 0) return false;
   if (!is_ragged(p) && ndq + nkv <= cus) return true;
-  return p->causal != 0 && ndq > 0 && nkv > 0 && ndq + nkv <= kFuseCausal * cus && ndq <= 4 * cus;
+  return p->causal != 0 && ndq > 0 && nkv > 0 && ndq + nkv <= kFuseCausal * cus &&
+         sigattn::dq_wave_pairs(p->B * p->H, p->Tq, p->Tk, true, is_ragged(p), cus);
 }
 
 // The recompute backward's dQ and dK/dV kernels run concurrently, dK/dV on a

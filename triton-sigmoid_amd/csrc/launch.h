@@ -26,9 +26,17 @@ inline bool fwd_wave_pairs(const KParams &p) {
   return (n == 1 ? 2 : 1) * n * p.B * p.H <= p.ncu;
 }
 
-// At most `per_cu` 128-row blocks per compute unit: where dQ does.
-inline bool wave_pairs(const KParams &p, int rows, int per_cu) {
-  return (int64_t)p.B * p.H * ((rows + 127) / 128) <= per_cu * (int64_t)p.ncu;
+// dQ, and with it the one-launch backward (capi.cpp's fuse_backward).  Dense
+// grids that, with dK/dV's, take at most one workgroup per CU keep one wave:
+// twice as many dQ workgroups share the dK/dV ones' CUs (fp16 B=2 T=1024 H=8
+// D=64 backward in one launch 28.1 / 26.8 us).  Other dense non-causal grids gain only where
+// they leave CUs idle; causal and ragged ones, which end with their longest
+// items, up to four blocks per CU.
+inline bool dq_wave_pairs(int64_t bh, int64_t Tq, int64_t Tk, bool causal, bool ragged, int64_t cus) {
+  const int64_t ndq = bh * ((Tq + 127) / 128), n = (Tk + 127) / 128;
+  if (!ragged && ndq + bh * n <= cus) return false;
+  if (!ragged && !causal) return ndq <= cus;
+  return ndq <= 4 * cus;
 }
 
 // Rows per workgroup and resident workgroups per CU of the MFMA forward and
@@ -56,9 +64,8 @@ void launch_bwd_dq_mfma(const KParams &p, int dtype, int D, bool causal, bool sc
 void launch_bwd_dkdv_mfma(const KParams &p, int dtype, int D, bool causal, bool scoremod,
                           bool dsout, hipStream_t st);
 // Both recompute kernels in one launch: the first B·H·ceil(Tk/128) workgroups
-// run dK/dV items, the rest dQ items (dense or padded problems, D <= 64, whose
-// dQ launch_bwd_dq_mfma runs in pairs of waves; bit-identical to
-// launch_bwd_dq_mfma + launch_bwd_dkdv_mfma).
+// run dK/dV items, the rest dQ items (dense or padded problems, D <= 64;
+// bit-identical to launch_bwd_dq_mfma + launch_bwd_dkdv_mfma).
 void launch_bwd_fused_mfma(const KParams &p, int dtype, int D, bool causal, bool scoremod, hipStream_t st);
 // dQ = dS·K·scale from the dS tiles a launch_bwd_dkdv_mfma(dsout = true) on
 // the same problem stored in p.ds (two-pass backward).
