@@ -30,13 +30,18 @@ inline bool fwd_wave_pairs(const KParams &p) {
 // grids that, with dK/dV's, take at most one workgroup per CU keep one wave:
 // twice as many dQ workgroups share the dK/dV ones' CUs (fp16 B=2 T=1024 H=8
 // D=64 backward in one launch 28.1 / 26.8 us).  Other dense non-causal grids gain only where
-// they leave CUs idle; causal and ragged ones, which end with their longest
-// items, up to four blocks per CU.
+// they leave CUs idle.  Causal and ragged grids end with their longest items,
+// so they gain up to four blocks per CU, fewer where the items are too short
+// to tell (n key blocks): backward, time of two waves over one, T=128 (n=1)
+// causal 1 / 1.5 / 2 blocks per CU 0.74 / 0.93 / 1.16, ragged 1 / 1.5 / 2
+// 1.01 / 1.07 / 1.14; T=512 (n=4) 2 / 3 / 4 0.80 / 1.04 / 1.01, causal dense
+// 0.96 / 0.91 / 0.98; T=700 (n=6) 3 / 4 0.98 / 1.05; T=2048 3 / 4 0.87 / 0.98.
 inline bool dq_wave_pairs(int64_t bh, int64_t Tq, int64_t Tk, bool causal, bool ragged, int64_t cus) {
   const int64_t ndq = bh * ((Tq + 127) / 128), n = (Tk + 127) / 128;
   if (!ragged && ndq + bh * n <= cus) return false;
   if (!ragged && !causal) return ndq <= cus;
-  return ndq <= 4 * cus;
+  const int64_t halves = n <= 2 ? (causal ? 3 : 2) : n <= 4 ? (ragged ? 4 : 6) : n <= 7 ? 6 : 8;  // of a block per CU
+  return 2 * ndq <= halves * cus;
 }
 
 // Rows per workgroup and resident workgroups per CU of the MFMA forward and
