@@ -651,3 +651,12 @@ def test_dq_wave_pairs_of_dense_grids_match_oracle(D, B, H, T, causal, with_mod)
                                   score_mod=None if mod is None else mod[b:b + 1])
         for name, x, want in zip(("dQ", "dK", "dV"), one, grads):
             assert_close_to_oracle(x[b:b + 1, :, h:h + 1], want, dtype, name)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T", [(15, 18, 33), (10, 18, 100), (15, 18, 100), (9, 12, 130)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fp32_short_padded_rows_match_oracle(D, B, H, T, causal):
+    """Short streamed rows: index order (WorkOrder's from 129 on) and one wave per
+    32 rows of D = 128 grids of more than half a block per compute unit."""
+    test_fp32_waves_per_rows_match_oracle(B, H, T, D, causal, False)

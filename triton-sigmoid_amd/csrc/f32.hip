@@ -556,12 +556,16 @@ template <int D, int WK> constexpr int bwd_f32_occupancy() { return D < 128 && W
 // dense ones from the last query or first key block.  occ: workgroups per CU.
 // Ragged, forward + backward, us, in index order / WorkOrder's: padded B=4
 // T=3000 H=8 D=64 1350 / 971, packed causal B=8 T=1500 H=8 D=128 949 / 726.
+// WorkOrder's passes over the batch, up to 4 us of every workgroup, need items
+// of some length: forward, time of index order over WorkOrder's, lengths T/4..T,
+// 0.75 to 2 blocks per CU: T=33 0.57-0.89, 128 0.71-1.05, 200 0.86-1.24, 384
+// 0.96-1.30, 512 0.99-1.37.
 // (Dense blocks of one head on one XCD, as the 16-bit kernels have them: B=2
 // T=1024 H=8 D=64 145 -> 152.)
 template <int WK, bool CAUSAL, bool ROWS_Q>
 __device__ __forceinline__ Item item_of(const KParams &p, int wg, int occ) {
   constexpr int RB = 32 * FW / WK;
-  if (p.ragged() && p.B <= 64) {
+  if (p.ragged() && p.B <= 64 && (ROWS_Q ? p.Tk : p.Tq) > 128) {
     const auto rows = [&](int i) SIGATTN_INLINE { return ROWS_Q ? p.len_q(i) : p.len_k(i); };
     const auto stream = [&](int i) SIGATTN_INLINE { return ROWS_Q ? p.len_k(i) : p.len_q(i); };
     const WorkItem it = CAUSAL ? WorkOrder::by_level(wg, p.B, p.H, rows, RB, p.nblk, ROWS_Q, p.ncu, occ)
@@ -822,12 +826,13 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
   add_waves<NDB, WK>(dva, lds, w, lane);
   add_waves<NDB, WK>(dka, lds, w, lane);
   if (wt == 0) rg.see(kf[0]), rg.see(vf[0]);
-  if (__syncthreads_or((wt == 0 && kok && (in_doubt(dva, 0x1p-88f, false) || in_doubt(dka, 0x1p-88f, false))) ||
-                       rg.wide(scale))) {
+  if (__syncthreads_or(rg.wide(scale) ||
+                       (wt == 0 && kok && (in_doubt(dva, 0x1p-88f, false) || in_doubt(dka, 0x1p-88f, false))))) {
     float least;
     bool zeros;
     const bool fits = doubt_below(rg, lds, least, zeros) && __builtin_fabsf(scale) < 0x1p32f;
-    if (__syncthreads_or(!fits || (wt == 0 && kok && (in_doubt(dva, least, zeros) || in_doubt(dka, least, zeros))))) {
+    if (__syncthreads_or(!fits ||
+                         (wt == 0 && kok && (in_doubt(dva, least, zeros) || in_doubt(dka, least, zeros))))) {
       dkdv_full<D, CAUSAL, SCOREMOD>(p, it, lds);
       return;
     }
