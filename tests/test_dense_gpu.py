@@ -660,3 +660,20 @@ def test_fp32_short_padded_rows_match_oracle(D, B, H, T, causal):
     """Short streamed rows: index order (WorkOrder's from 129 on) and one wave per
     32 rows of D = 128 grids of more than half a block per compute unit."""
     test_fp32_waves_per_rows_match_oracle(B, H, T, D, causal, False)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,T", [(10, 18, 100), (10, 14, 200), (5, 9, 400)])  # 180, 280 and 180 blocks of 128 rows
+@pytest.mark.parametrize("causal", [False, True])
+def test_fp32_dense_waves_per_rows_match_oracle(D, B, H, T, causal):
+    dtype = torch.float32
+    q, k, v, do = _inputs(B, T, H, D, dtype, seed=T + D)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    o = ts.sigmoid_attention(q, k, v, is_causal=causal, sigmoid_bias=-2.0)
+    o.backward(do)
+    for b, h in ((0, H - 1), (B - 1, 0)):
+        one = [t.detach()[b:b + 1, :, h:h + 1] for t in (q, k, v, do)]
+        want_o, grads = oracle_fwd_bwd(*one, scale=np.float32(1.0 / math.sqrt(D)), bias=np.full(1, -2.0), causal=causal)
+        for name, got, want in zip(("O", "dQ", "dK", "dV"), (o, q.grad, k.grad, v.grad), (want_o, *grads)):
+            assert_close_to_oracle(got[b:b + 1, :, h:h + 1], want, dtype, name)

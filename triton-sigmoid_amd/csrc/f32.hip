@@ -854,21 +854,30 @@ __global__ __launch_bounds__(64 * FW, (bwd_f32_occupancy<D, WK>())) void dkdv_f3
 // D=128, 2048 blocks, 7016 / 7780 (10357).  Four waves pay where their blocks of
 // 32 rows leave CUs idle (B=2 T=256 H=4 D=64: kernels 25 + 32 + 40 -> 12 + 15 +
 // 16 us); 128 rows of three parts of two tensors do not fit at D = 128.
-template <int D> int f32_waves_per_rows(const KParams &p, int rows) {
-  const int64_t bh = (int64_t)p.B * p.H;
-  if (D < 128 && bh * ((rows + 31) / 32) <= p.ncu) return 4;
-  return bh * ((rows + 127) / 128) < 2 * (int64_t)p.ncu ? 2 : 1;
+// At D = 128 two waves need the whole CU, so more than half a block per CU of
+// them is two rounds: worth it where the items differ and are long.  Time of
+// WK = 1 over 2, 0.75 to 1.5 blocks per CU, forward / dQ and dK/dV: T=100 0.69-0.93 /
+// 0.76-1.0 (D = 64, from 1.25: 0.77-0.97 / 0.79-0.93), dense non-causal T=200 to
+// 512 0.71-1.00 / 0.75-1.08, causal T=512 1.04-1.55 / 0.89-1.27; T=33 0.9-1.2.
+template <int D> int f32_waves_per_rows(const KParams &p, int rows, int stream, bool causal) {
+  const int64_t bh = (int64_t)p.B * p.H, blocks = bh * ((rows + 127) / 128), cus = p.ncu;
+  if (D < 128 && bh * ((rows + 31) / 32) <= cus) return 4;
+  if (D == 128 && stream <= 128 && blocks > cus) return 1;
+  if (D >= 64 && stream > 64 && (D == 128 ? 2 : 1) * blocks > cus &&
+      (stream <= 128 || (D == 128 && !causal && !p.ragged() && (stream <= 256 || blocks <= cus))))
+    return 1;
+  return blocks < 2 * cus ? 2 : 1;
 }
 
 // Calls launch(std::integral_constant<int, WK>, p, workgroups) with p.nblk set.
-template <int D, class F> void by_waves(const KParams &kp, int rows, F &&launch) {
+template <int D, class F> void by_waves(const KParams &kp, int rows, int stream, bool causal, F &&launch) {
   KParams p = kp;
   const auto go = [&](auto wk) {
     constexpr int RB = 32 * FW / decltype(wk)::value;
     p.nblk = (rows + RB - 1) / RB;
     launch(wk, p, (int64_t)p.nblk * p.B * p.H);
   };
-  switch (f32_waves_per_rows<D>(p, rows)) {
+  switch (f32_waves_per_rows<D>(p, rows, stream, causal)) {
     case 4:
       if constexpr (D < 128) return go(std::integral_constant<int, 4>{});
       break;
@@ -879,7 +888,7 @@ template <int D, class F> void by_waves(const KParams &kp, int rows, F &&launch)
 }
 
 template <int D> void fwd_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  by_waves<D>(kp, kp.Tq, [&](auto wk, const KParams &p, int64_t n) {
+  by_waves<D>(kp, kp.Tq, kp.Tk, causal, [&](auto wk, const KParams &p, int64_t n) {
     constexpr int WK = decltype(wk)::value;
     const dim3 grid((unsigned)(n + p.ngap[0] + p.ngap[1])), block(64 * FW);
     if (causal) {
@@ -893,7 +902,7 @@ template <int D> void fwd_t(const KParams &kp, bool causal, bool scoremod, hipSt
 }
 
 template <int D> void dq_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  by_waves<D>(kp, kp.Tq, [&](auto wk, const KParams &p, int64_t n) {
+  by_waves<D>(kp, kp.Tq, kp.Tk, causal, [&](auto wk, const KParams &p, int64_t n) {
     constexpr int WK = decltype(wk)::value;
     const dim3 grid((unsigned)(n + p.ngap[0] + p.ngap[1])), block(64 * FW);
     if (causal) {
@@ -907,7 +916,7 @@ template <int D> void dq_t(const KParams &kp, bool causal, bool scoremod, hipStr
 }
 
 template <int D> void dkdv_t(const KParams &kp, bool causal, bool scoremod, hipStream_t st) {
-  by_waves<D>(kp, kp.Tk, [&](auto wk, const KParams &p, int64_t n) {
+  by_waves<D>(kp, kp.Tk, kp.Tq, causal, [&](auto wk, const KParams &p, int64_t n) {
     constexpr int WK = decltype(wk)::value;
     const dim3 grid((unsigned)n), block(64 * FW);  // no gap rows here (the dQ launch's)
     if (causal) {
