@@ -84,8 +84,8 @@ bool use_mfma(const sigattn_problem *p, const void *const *ptrs, int nptr) {
   return rows_dma_ready(p, ptrs, nptr, 2);
 }
 
-// True when the fp32 MFMA kernels (v_mfma_f32_32x32x2_f32) can take the
-// problem: fp32, D of 16, 32, 64 or 128, rows as rows_dma_ready requires.
+// True when the fp32 MFMA kernels (three-part bf16 splits, see f32.hip) can take
+// the problem: fp32, D of 16, 32, 64 or 128, rows as rows_dma_ready requires.
 bool use_f32_mfma(const sigattn_problem *p, const void *const *ptrs, int nptr) {
   if (p->dtype != SIGATTN_F32 || !is_pow2_head_dim(p->D)) return false;
   return rows_dma_ready(p, ptrs, nptr, 4);

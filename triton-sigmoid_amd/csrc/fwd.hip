@@ -8,11 +8,12 @@
 //   I/O dtype; O += P·V in fp32; O is stored in the I/O dtype; query rows at or
 //   past seq_lens_q are zero; keys at or past seq_lens_k get P = 0.
 //
-// Structure: one workgroup = 256 queries of one (batch, head), split over its
-// waves (NCB 32-row MFMA column blocks per wave; with NCB = 2 every K or Vᵀ
-// operand read from LDS feeds two MFMAs).
-//   * K and V stream through a 4-stage ring of 64-key swizzled LDS tiles
-//     filled by direct global->LDS copies one tile ahead;
+// Structure: one workgroup = 256 queries of one (batch, head) at D = 128, 64 to
+// 256 at D <= 64 (launch_fwd_t), split over its waves (NCB 32-row MFMA column
+// blocks per wave; with NCB = 2 every K or Vᵀ operand read from LDS feeds two
+// MFMAs; with WK = 2 two waves share each 32 queries).
+//   * K and V stream through a ring of three or four 64-key swizzled LDS tiles
+//     (fwd_stages) filled by direct global->LDS copies one tile ahead;
 //   * keys are processed as a continuous sequence of 32-key blocks g with a
 //     three-deep software pipeline: region r issues the Sᵀ(r) = K·Qᵀ MFMA
 //     chains and the Oᵀ += Vᵀ·Pᵀ(r-2) MFMAs while the VALU computes
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK, NCB>())) void fwd_m
   // score_mod, which spills at four waves per SIMD otherwise).
   constexpr int LA = D == 128 ? (SCOREMOD ? 8 : 16) : (D == 32 && SCOREMOD ? 2 : 4);
   constexpr int NWD = 8 * NCB;          // packed P words per block
-  constexpr int BAR = NSTEP - LA;       // step of the tile barrier in odd regions
+  constexpr int BAR = NSTEP - LA;       // step of the tile barrier (in odd regions; WK = 2: in all)
   static_assert(NSTEP % LA == 0, "region shape");
 
   __shared__ __attribute__((aligned(16))) uint16_t sK[NST][BN * D];
@@ -276,19 +277,23 @@ __global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK, NCB>())) void fwd_m
     // 32-key block that the wave's region r computes S of.
     auto block_of = [&](int r) SIGATTN_INLINE { return WK == 2 ? 2 * r + wt : r; };
 
-    // Region r (U = r mod 8, so every slot and ring stage is static):
+    // Region r (U = r modulo the regions of a ring turn, so every slot and ring
+    // stage is static):
     //   MFMA: Sᵀ(r) = K·Qᵀ and Oᵀ += Vᵀ·Pᵀ(r-2), one step = NCB MFMAs (one per
     //         column block) sharing an A operand read LA steps earlier;
     //   VALU: P(r-1) = sigmoid(Sᵀ(r-1)) as a two-stage pipeline over packed
     //         words (exp2 of the next word, then reciprocal and packing);
     //   LDS:  the operand LA steps ahead (wrapping into region r+1).
-    // Block g lives in tile g/2 (rows 32*(g%2)) in ring stage (g/2)%4.  In odd
+    // Block g lives in tile g/2 (rows 32*(g%2)) in ring stage (g/2)%NST.  In odd
     // regions r = 2u-1, step BAR publishes tile u (its first read, the K rows of
     // block r+1, comes next) and starts the copy of tile u+1 into the stage of
     // tile u+1-NST.  With four stages that tile's last reads were issued two
     // regions earlier, so the barrier needs no wait for this wave's own LDS
     // reads; with three (D = 64) they were issued in this region, and every
     // wave waits for them before the barrier.
+    // WK = 2: region r is the wave's block of tile r (stage r%4), so step BAR of
+    // every region publishes tile r+1 and starts the copy of tile r+2 into the
+    // stage of tile r-2, whose Vᵀ operands this region reads: the same wait.
     auto region = [&](int r, auto u_tag) SIGATTN_INLINE {
       constexpr int U = decltype(u_tag)::value;
       constexpr int SL = U % 2;                    // parity of blocks r and r-2
@@ -386,7 +391,8 @@ __global__ __launch_bounds__(64 * NWV, (fwd_occupancy<D, WK, NCB>())) void fwd_m
     // Pipeline fill: Pᵀ(-2) = Pᵀ(-1) = 0 (the latter through its mask).  The
     // Vᵀ operands of blocks -2 and -1 come from ring stage NST-1, zeroed here
     // (tile NST-1 is copied into it from the barrier of region 2·NST-5 on,
-    // after every read of blocks -2 and -1), so 0 * operand stays 0.
+    // after every read of blocks -2 and -1), so 0 * operand stays 0.  WK = 2:
+    // from stages NST-2 and NST-1, refilled in regions 0 and 1.
   #pragma unroll
     for (int x = 0; x < 2; ++x) {
   #pragma unroll

@@ -78,13 +78,14 @@ void launch_bwd_dq_ds_mfma(const KParams &p, int dtype, int D, bool causal, hipS
 
 // Split-KV forward (decode shapes: Tq <= 32, non-causal) with the MFMA
 // kernels' requirements; p.nsplit / p.chunk set, p.ws holds
-// nsplit * B * H * Tq * D floats when nsplit > 1.
+// nsplit * B * H * Tq * D floats when nsplit > 1 (p.rows > 0: rows * H * Tq * D
+// and 2 * B ints).
 void launch_fwd_splitkv(const KParams &p, int dtype, int D, bool scoremod, hipStream_t st);
 
 // Fixed device scratch of the split-KV forward for callers that cannot
 // allocate (sigattn_fwd_noalloc): a file-scope __device__ array of this many
-// bytes in decode.hip, one per GPU, held until the process ends.  The split
-// plan never needs more: fp32 partials of nsplit * B * H * Tq * D floats with
+// bytes in decode.hip, one per GPU, held until the process ends.  Its plan (the
+// shared form's) never needs more: fp32 partials of nsplit * B * H * Tq * D floats with
 // nsplit * B * H < 1024 (splitting stops at 512 (batch, head) pairs), Tq <= 32
 // and D <= 128 stay below 16 MiB.
 constexpr size_t kSplitScratchBytes = size_t(16) << 20;
