@@ -541,8 +541,9 @@ DECODE_CONFIGS = [
 
 def decode_bench(iters: int = 20):
     """Split-KV forward at decode shapes through the C ABI: average kernel time
-    (the chunk kernel and the partial sum) with the workspace the library asks
-    for, and with none (one chunk per (batch, head)), on torch's current stream
+    (the chunk kernel and the partial sum) by the plan the public APIs launch
+    (sigattn_fwd_decode), by sigattn_fwd_ws with the workspace it asks for, and
+    with none (one chunk per (batch, head)), on torch's current stream
     between HIP events.  The kernel is HBM-bound: its algorithmic traffic is
     K and V of the valid cache (2 * D * 2 bytes per key, batch and head) plus
     Q and O."""
@@ -568,14 +569,17 @@ def decode_bench(iters: int = 20):
         pr = _capi._problem(q, k, v, bias, None, scale, sq, sk, False)
         out = torch.empty_like(q)
         nbytes = int(lib.sigattn_fwd_workspace_bytes(ctypes.byref(pr)))
-        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+        dbytes = int(lib.sigattn_fwd_decode_workspace_bytes(ctypes.byref(pr)))
+        ws = torch.empty(max(nbytes, dbytes, 16), dtype=torch.uint8, device=dev)
         stream = torch.cuda.current_stream().cuda_stream
         kv_keys = int(lens.sum())
         traffic = 2 * D * 2 * kv_keys * H + 2 * B * Tq * H * D * 2
         flops = 4 * D * Tq * kv_keys * H
-        row = dict(cfg, workspace_bytes=nbytes)
-        for name, wptr, wbytes in (("split", ws.data_ptr() if nbytes else None, nbytes), ("one_chunk", None, 0)):
-            call = lambda: lib.sigattn_fwd_ws(ctypes.byref(pr), out.data_ptr(), wptr, wbytes, stream)
+        row = dict(cfg, workspace_bytes=nbytes, decode_workspace_bytes=dbytes)
+        for name, fwd, wbytes in (("decode", lib.sigattn_fwd_decode, dbytes), ("split", lib.sigattn_fwd_ws, nbytes),
+                                  ("one_chunk", lib.sigattn_fwd_ws, 0)):
+            wptr = ws.data_ptr() if wbytes else None
+            call = lambda: fwd(ctypes.byref(pr), out.data_ptr(), wptr, wbytes, stream)
             for _ in range(3):
                 assert call() == 0
             torch.cuda.synchronize()
@@ -590,7 +594,7 @@ def decode_bench(iters: int = 20):
                              hbm_frac=round(traffic / ms / 1e6 / (HBM_PEAK_TBPS * 1e3), 4),
                              tflops=round(flops / ms / 1e9, 1))
         rows.append(row)
-        log(f"[decode] {cfg}: split {row['split']} | one chunk {row['one_chunk']}")
+        log(f"[decode] {cfg}: decode {row['decode']} | split {row['split']} | one chunk {row['one_chunk']}")
         del q, k, v, out, ws
         torch.cuda.empty_cache()
     return rows

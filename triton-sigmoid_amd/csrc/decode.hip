@@ -77,7 +77,8 @@ hipError_t splitkv_scratch(float **ptr) {
 // of one (batch, head)):
 //   * WPU = 4: the workgroup's waves take every fourth 32-key block of its
 //     chunk and add their partials through LDS -- short caches, where there
-//     are too few chunks to give every wave one of its own;
+//     are too few chunks to give every wave one of its own, or too few bytes to
+//     pay for partials and a second launch;
 //   * WPU = 1: every wave has a unit of its own, the units of one key range
 //     in head order, so the four waves of a workgroup read the rows of four
 //     neighbouring heads (4 * 2 * D contiguous bytes of every [B, T, H, D]
@@ -93,7 +94,8 @@ hipError_t splitkv_scratch(float **ptr) {
 //     launches); one-wave workgroups on the heads of one XCD took 348, 364 and
 //     214 us, two-wave ones 317, 317 and 191.
 //     Ragged caches would leave such units uneven, so the device cuts the
-//     sequences (WaveUnits): p.rows chunks in all, of about equal length.
+//     sequences of batches of up to 64 (WaveUnits): p.rows chunks in all, of
+//     about equal length.
 // A wave's K and V blocks have two stages each; the K stage is refilled as
 // soon as S is computed and the V stage after the output product, so three of
 // the four blocks are in flight at any time.
