@@ -168,8 +168,8 @@ def test_decode_long_cache_sum_of_halves():
     (8, 16, 32, 8200, 64, False, True),    # all 32 query rows
     (9, 16, 2, 3001, 128, True, True),     # packed rows
     (16, 128, 2, 300, 64, False, False),   # one chunk per (batch, head): no partials
-    (64, 16, 1, 700, 64, False, False),    # a batch per lane, 2 rows of partials each
-    (65, 16, 1, 700, 64, False, False),    # one more: chunks of one length for all
+    (64, 16, 1, 2100, 64, False, False),   # a sequence per lane, 2 rows of partials each
+    (65, 16, 1, 2100, 64, False, False),   # one more: chunks of one length for all
     (12, 16, 32, 12000, 64, False, False), # keys for one round of waves, not for two
     (3, 16, 1, 30000, 128, False, True),   # ... and long sequences
 ])
@@ -285,9 +285,8 @@ def test_batches_of_more_than_a_lane_each_take_an_odd_number_of_chunks(B, H, Tq,
 
 
 @pytest.mark.parametrize("B,H,Tq,Tk,D,packed,mod", [
-    (64, 16, 1, 2100, 64, False, True),   # a sequence per lane
-    (65, 16, 1, 2100, 64, False, True),   # one more: chunks of one length for all
-    (72, 8, 2, 2600, 128, True, False),   # ... five of them, packed rows
+    (65, 16, 1, 2100, 64, False, True),   # three chunks of one length for all
+    (72, 8, 2, 2600, 128, True, False),   # five, packed rows
     (80, 4, 1, 6000, 64, False, False),
 ])
 def test_decode_large_batches_match_the_general_path(B, H, Tq, Tk, D, packed, mod):

@@ -552,7 +552,7 @@ def test_fp32_tiny_operands_of_ordinary_results_match_the_portable_kernels(D, B,
         assert torch.all((x - y).abs() <= bound * top), (name, ((x - y).abs() / top).max().item())
 
 
-# --- D <= 64 forward and dQ: two waves per 32 rows on small grids, one on large ones ---
+# --- D <= 64 forward and dQ: two waves per 32 rows on small grids, one on larger ones ---
 
 @pytest.mark.parametrize("D", [16, 32, 64])
 @pytest.mark.parametrize("T", [63, 65, 96, 129, 257, 321])
@@ -560,8 +560,8 @@ def test_fp32_tiny_operands_of_ordinary_results_match_the_portable_kernels(D, B,
 @pytest.mark.parametrize("layout", ["dense", "mod", "padded"])
 def test_wave_pairs_and_single_waves_match_oracle(D, T, causal, layout):
     """17 x 64 (batch, head) pairs are more than four blocks per compute unit
-    (a wave per 32 rows, per 64 at D = 64); one pair alone is a small grid (two
-    waves per 32 rows).  Both against the oracle, on remainders of 32-, 64-,
+    (a wave per 32 rows); one pair alone is a small grid (two waves per 32 rows in
+    the forward and, padded, in dQ).  Both against the oracle, on remainders of 32-, 64-,
     128- and 256-row blocks."""
     B, H, dtype = 17, 64, torch.bfloat16
     q, k, v, do = _inputs(B, T, H, D, dtype, seed=T + D)

@@ -430,7 +430,8 @@ def test_default_bias_kernel_equals_the_operators(B):
 @pytest.mark.parametrize("padded", [False, True])
 def test_one_launch_causal_backward_equals_the_two_kernels(D, B, H, T, padded):
     """Causal dense and padded grids run dK/dV and dQ in one launch up to six
-    128-row blocks per compute unit: the same bits as the kernels apart."""
+    128-row blocks per compute unit (fewer of short sequences): the same bits as
+    the kernels apart."""
     g = torch.Generator().manual_seed(T + D)
     q, k, v, do = (randn((B, T, H, D), torch.bfloat16, DEV, g) for _ in range(4))
     lens = torch.randint(0, T + 1, (B,), generator=g, dtype=torch.int32).to(DEV) if padded else None
